@@ -365,6 +365,46 @@ def test_quantize_bit_exact(kind, src):
     np.testing.assert_array_equal(deq, O.dequantize(rc, rs, kind).astype(np.float32))
 
 
+@pytest.mark.parametrize("kind", ["i8", "q4"])
+@pytest.mark.parametrize("src", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,D,offset", [(1, 8, 0), (17, 64, 0), (33, 136, 0), (250, 392, 0), (50, 512, 0), (19, 1024, 0),
+                                           (19, 1032, 0), (40, 384, 1), (21, 70, 0)])
+def test_quantize_widths_and_special_values(kind, src, rows, D, offset):
+    """Widths at the edges of the register layouts and outside them, a source off its alignment, rows of one value,
+    of ties, of the halfway points between codes, beyond the scale's range, with infinities and NaN."""
+    rng = np.random.default_rng(rows * D)
+    t = (rng.standard_normal((rows, D)) * 10.0 ** rng.integers(-7, 4, (rows, 1))).astype(np.float32)
+    lo = -128 if kind == "i8" else -8
+    if rows > 16:
+        t[2] = 3.0                                                      # every column ties
+        t[3] = (rng.integers(2 * lo, -2 * lo, D) / 2).astype(np.float32)      # halves: ties of the rounding
+        t[3, D // 2] = lo
+        t[4, 1] = 3e38                                                  # the scale overflows fp16
+        t[5] = 1e-9                                                     # the scale underflows to zero
+        t[6] = -4e-6                                                    # the scale is subnormal in fp16
+        t[7, 2], t[8, 3], t[9] = np.inf, np.nan, np.nan
+    tt = torch.from_numpy(t)
+    if src == "bf16":
+        bits = O.bf16_bits_rtne(np.where(np.isnan(t), 0, t).astype(np.float32))
+        tt, t = bf16_from_bits(bits), O.bf16_to_f32(bits)
+    buf = torch.zeros(rows * D + offset, dtype=tt.dtype, device=DEV)
+    x = buf[offset:].view(rows, D)
+    x.copy_(tt)
+    codes, sc = (K.quantize_int8 if kind == "i8" else K.quantize_q4)(x)
+    # what the oracle's numpy leaves open for rows with a NaN: it does not count as the largest magnitude (a row of
+    # NaN alone has a NaN scale), and its code is the lowest
+    with np.errstate(all="ignore"):
+        m = t[np.arange(rows), np.where(np.isnan(t), -1, np.abs(t)).argmax(1)]
+        rs = (m / np.float32(lo)).astype(np.float16)
+        rs = np.where(rs == 0, np.float16(1), rs)
+        c = np.rint(t / rs.astype(np.float32)[:, None])
+    c = np.clip(np.where(np.isnan(c), lo, c), lo, -lo - 1).astype(np.int64)
+    rc = c.astype(np.int8) if kind == "i8" else ((c[:, :D // 2] + 8) | (c[:, D // 2:] + 8) << 4).astype(np.uint8)
+    got = sc.cpu().numpy()
+    assert np.array_equal(np.isnan(got), np.isnan(rs)) and np.array_equal(got[~np.isnan(rs)], rs[~np.isnan(rs)])
+    assert np.array_equal(codes.cpu().numpy(), rc)
+
+
 def test_quantize_golden():
     with open(os.path.join(GOLDEN, "quant_known.json")) as f:
         g = json.load(f)
