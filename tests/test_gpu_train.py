@@ -329,6 +329,38 @@ def test_lazy_adam_fp32_bit_exact(rows, D):
         assert not Tt.cpu().any()
 
 
+@pytest.mark.parametrize("state", ["fp32", "bf16", "int8"])
+@pytest.mark.parametrize("rows,D,read", [(1, 4, 1.0), (65, 24, 0.5), (70001, 24, 0.01), (70001, 24, 0.9), (131, 28, 0.7),
+                                         (90, 64, 1.0), (70, 68, 0.5), (33, 128, 0.6), (600000, 8, 0.3)])
+def test_lazy_adam_narrow_rows_bit_exact(state, rows, D, read):
+    """Tables of up to 128 columns: widths that fill their lane group and that leave lanes idle, one and several rows
+    per scan, few and most of the rows flagged, the last scan cut off by the table's end."""
+    note(f"lazy adam narrow {state} rows={rows} D={D} read={read}")
+    rng, p = _adam_case(rows, D, rows + 3 * D)
+    mdt, vdt = {"fp32": (torch.float32,) * 2, "bf16": (torch.bfloat16,) * 2, "int8": (torch.int8, torch.uint8)}[state]
+    M, V = torch.zeros(rows, D, dtype=mdt, device=DEV), torch.zeros(rows, D, dtype=vdt, device=DEV)
+    MS, VS = torch.zeros(rows, device=DEV), torch.zeros(rows, device=DEV)
+    m, v = (a.float().cpu().numpy() if state != "int8" else a.cpu().numpy() for a in (M, V))
+    ms, vs = (np.zeros(rows, np.float32) for _ in range(2))
+    P = torch.from_numpy(p.copy()).to(DEV)
+    for step in range(1, 3):
+        acc = (rng.standard_normal((rows, D)) * 1e-2).astype(np.float32)
+        touched = rng.random(rows) < read
+        touched[-1] = True
+        A, Tt = torch.from_numpy(acc.copy()).to(DEV), torch.from_numpy(touched.copy()).to(DEV)
+        hyper = (step, 1e-3, 0.9, 0.95, 1e-8)
+        if state == "fp32":
+            KR.lazy_adam_step(P, M, V, A, Tt, 0.5, *hyper)
+            p, m, v, acc_r, _ = T.lazy_adam(p, m, v, acc, touched, 0.5, *hyper)
+        else:
+            KR.lazy_adam_step_lowmem(P, M, V, A, Tt, 0.5, *hyper, state, *((MS, VS) if state == "int8" else ()))
+            p, m, v, ms, vs, acc_r, _ = T.lazy_adam_lowmem(p, m, v, ms, vs, acc, touched, 0.5, *hyper, state == "int8")
+        for got, ref in ((P, p), (M, m), (V, v), (A, acc_r), (MS, ms), (VS, vs)):
+            if ref is not None:
+                np.testing.assert_array_equal(got.float().cpu().numpy(), np.asarray(ref, np.float32))
+        assert not Tt.cpu().any()
+
+
 @pytest.mark.parametrize("state,rows,D", [("bf16", 200, 384), ("int8", 200, 384), ("int8", 33, 100),
                                           ("bf16", 30, 130), ("int8", 30, 98), ("int8", 40, 512), ("int8", 50, 300), ("bf16", 45, 300)])
 def test_lazy_adam_lowmem_bit_exact(state, rows, D):
