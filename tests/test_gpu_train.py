@@ -302,6 +302,30 @@ def test_bag_backward_sorted_workspace_checks():
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("rows,D,read,offset", [(1, 1, 1.0, 0), (5, 24, 0.0, 0), (64, 384, 1.0, 0), (300, 384, 0.4, 0), (257, 260, 0.5, 0),
+                                                (1000, 7, 0.3, 0), (130, 512, 0.5, 1), (70000, 24, 0.02, 0),
+                                                (1100000, 8, 0.5, 0)])
+def test_flagged_norm(rows, D, read, offset):
+    """The norm over the flagged rows in fp64, rounded twice to fp32 (its sum and its root): the same value within two
+    roundings, whatever the unflagged rows hold, and the same on every call."""
+    note(f"flagged norm rows={rows} D={D} read={read} offset={offset}")
+    g = torch.Generator(device=DEV).manual_seed(rows + D)
+    buf = torch.empty(rows * D + offset, device=DEV)
+    acc = buf[offset:].view(rows, D).normal_(generator=g)
+    touched = torch.rand(rows, device=DEV, generator=g) < read
+    acc[~touched] = float("nan")
+    got = KR.flagged_norm(acc, touched)
+    ref = acc[touched].double().norm().item()
+    assert abs(got.item() - ref) <= 2 ** -23 * ref
+    assert all(torch.equal(KR.flagged_norm(acc, touched), got) for _ in range(3))
+    if touched.any():
+        row = int(touched.nonzero()[-1])
+        acc[row, -1] = float("inf")
+        assert KR.flagged_norm(acc, touched).item() == float("inf")
+        acc[row, 0] = float("nan")
+        assert D == 1 or torch.isnan(KR.flagged_norm(acc, touched))
+
+
 def _adam_case(rows, D, seed):
     rng = np.random.default_rng(seed)
     p = rng.standard_normal((rows, D)).astype(np.float32)
