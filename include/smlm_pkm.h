@@ -469,6 +469,29 @@ int smlm_engram_hash(const int64_t *c, int64_t B, int64_t T, int64_t c_len, cons
 int smlm_row_gather(const int64_t *rows, int64_t M, const void *table, int table_dtype, int64_t table_rows, int D,
                     void *out, void *stream);
 
+/*
+ * The Engram module behind its projections (smlm/engram.py:119-131) in one launch:
+ *   a = sigmoid(<RMSNorm(h; wh), RMSNorm(k; wk)> / sqrt(d)),  gv = a v,  u = RMSNorm(gv; wv) rounded to bf16,
+ *   c_t = sum_i conv[:, 0, i] u_(t - (taps - 1 - i) dilation),  y = silu(c) + gv
+ * h, y (B, T, d) of h_dtype, k, v (B, T, d) bf16, wh, wk, wv (d,) and conv (d, 1, taps) of h_dtype (SMLM_BF16 or
+ * SMLM_F32); left (B, past, d) bf16 or NULL (zeros): the u before the sequence, past = (taps - 1) * dilation; tail
+ * (B, past, d) bf16 or NULL: receives the last `past` u of left and the sequence together.  Arithmetic in fp32.
+ * d a multiple of 8 up to 512, taps <= 4, past <= 32; every tensor but conv 16-byte aligned.
+ */
+int smlm_engram_mix(const void *h, const void *k, const void *v, const void *wh, const void *wk, const void *wv,
+                    const void *conv, int h_dtype, const void *left, void *tail, int64_t B, int64_t T, int d, int taps,
+                    int dilation, float eps, void *y, void *stream);
+
+/*
+ * Its gradient for h_dtype SMLM_F32 and no left: from gy (B, T, d) fp32, dh fp32, dk and dv bf16, and the weights'
+ * gradients fp32, summed in a fixed order.  parts: caller-owned scratch of smlm_engram_mix_parts floats.
+ */
+int64_t smlm_engram_mix_parts(int64_t B, int64_t T, int d, int taps);
+int smlm_engram_mix_backward(const float *gy, const float *h, const void *k, const void *v, const float *wh,
+                             const float *wk, const float *wv, const float *conv, int64_t B, int64_t T, int d, int taps,
+                             int dilation, float eps, float *dh, void *dk, void *dv, float *dwh, float *dwk, float *dwv,
+                             float *dconv, float *parts, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -69,6 +69,9 @@ EXPORTS = {
     "smlm_flagged_norm_parts": (_i, []),
     "smlm_flagged_norm": (_i, [_p, _p, _i64, _i, _p, _p, _p]),
     "smlm_engram_hash": (_i, [_p, _i64, _i64, _i64, _p, _p, _i, _i, _i, _i64, _p, _p]),
+    "smlm_engram_mix": (_i, [_p] * 7 + [_i, _p, _p, _i64, _i64, _i, _i, _i, _f, _p, _p]),
+    "smlm_engram_mix_parts": (_i64, [_i64, _i64, _i, _i]),
+    "smlm_engram_mix_backward": (_i, [_p] * 8 + [_i64, _i64, _i, _i, _i, _f] + [_p] * 9),
     "smlm_row_gather": (_i, [_p, _i64, _p, _i, _i64, _i, _p, _p]),
 }
 ADAM_F32, ADAM_BF16, ADAM_INT8 = 0, 1, 2

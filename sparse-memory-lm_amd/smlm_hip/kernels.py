@@ -942,3 +942,69 @@ def row_gather(rows, table):
                                     table.shape[0], table.shape[1], out.data_ptr(), _stream(table))
     _lib.check(rc, "smlm_row_gather")
     return out.view(*rows.shape, table.shape[1])
+
+
+ENGRAM_MIX_MAX_D, ENGRAM_MIX_MAX_TAPS, ENGRAM_MIX_MAX_PAST = 512, 4, 32     # csrc/engram_mix.hip
+
+
+def _aligned(t):
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _engram_mix_args(name, h, k, v, weights, conv, dilation):
+    _need_cuda(name, h, k, v, conv, *weights)
+    if h.dim() != 3 or k.shape != h.shape or v.shape != h.shape or h.dtype not in _DT or k.dtype != torch.bfloat16 \
+            or v.dtype != torch.bfloat16:
+        raise ValueError(f"{name}: h (B, T, d) bf16 or fp32 and k, v of its shape in bf16")
+    d = h.shape[2]
+    if any(w.shape != (d,) or w.dtype != h.dtype for w in weights) or conv.dim() != 3 or conv.shape[:2] != (d, 1) \
+            or conv.dtype != h.dtype:
+        raise ValueError(f"{name}: norm weights ({d},) and conv ({d}, 1, taps) of h's dtype")
+    return [_aligned(t) for t in (h, k, v, *weights)] + [conv.contiguous(), (conv.shape[2] - 1) * dilation]
+
+
+def engram_mix(h, k, v, wh, wk, wv, conv, dilation, eps, left=None, keep_tail=False):
+    """The Engram module behind its projections (smlm/engram.py:119-131) in one launch (smlm_engram_mix): gate
+    a = sigmoid(<RMSNorm(h), RMSNorm(k)> / sqrt(d)), gv = a v, causal depthwise convolution of u = RMSNorm(gv), and
+    silu(conv) + gv.  h (B, T, d) bf16 or fp32, k, v bf16, norm weights (d,) and conv (d, 1, taps) of h's dtype; left
+    (B, past, d) bf16: the u before the sequence (None: zeros).  Returns y (B, T, d) of h's dtype, with keep_tail
+    (y, tail), tail (B, past, d) the last `past` u.  Forward only."""
+    h, k, v, wh, wk, wv, conv, past = _engram_mix_args("engram_mix", h, k, v, (wh, wk, wv), conv, dilation)
+    B, T, d = h.shape
+    if left is not None:
+        _need_cuda("engram_mix", left)
+        if left.dtype != torch.bfloat16 or tuple(left.shape) != (B, past, d):
+            raise ValueError(f"engram_mix: left must be ({B}, {past}, {d}) bf16")
+        left = _aligned(left)
+    y = torch.empty_like(h)
+    tail = torch.empty(B, past, d, dtype=torch.bfloat16, device=h.device) if keep_tail else None
+    rc = _lib.lib().smlm_engram_mix(
+        h.data_ptr(), k.data_ptr(), v.data_ptr(), wh.data_ptr(), wk.data_ptr(), wv.data_ptr(), conv.data_ptr(),
+        _DT[h.dtype], left.data_ptr() if left is not None else None, tail.data_ptr() if keep_tail and past else None,
+        B, T, d, conv.shape[2], dilation, eps, y.data_ptr(), _stream(h))
+    _lib.check(rc, "smlm_engram_mix")
+    return (y, tail) if keep_tail else y
+
+
+def engram_mix_backward(gy, h, k, v, wh, wk, wv, conv, dilation, eps):
+    """The gradients of engram_mix(h fp32, ...) without left (smlm_engram_mix_backward): (dh fp32, dk, dv bf16, dwh,
+    dwk, dwv, dconv fp32) from gy (B, T, d) fp32.  The same result on every call."""
+    h, k, v, wh, wk, wv, conv, _ = _engram_mix_args("engram_mix_backward", h, k, v, (wh, wk, wv), conv, dilation)
+    if h.dtype != torch.float32 or gy.dtype != torch.float32 or gy.shape != h.shape:
+        raise ValueError("engram_mix_backward: gy and h must be fp32 of one shape")
+    _need_cuda("engram_mix_backward", gy)
+    gy = _aligned(gy)
+    B, T, d = h.shape
+    taps = conv.shape[2]
+    L = _lib.lib()
+    dh, dk, dv = torch.empty_like(h), torch.empty_like(k), torch.empty_like(v)
+    dw = torch.empty(3, d, dtype=torch.float32, device=h.device)
+    dconv = torch.empty_like(conv)
+    parts = torch.empty(max(L.smlm_engram_mix_parts(B, T, d, taps), 1), dtype=torch.float32, device=h.device)
+    rc = L.smlm_engram_mix_backward(
+        gy.data_ptr(), h.data_ptr(), k.data_ptr(), v.data_ptr(), wh.data_ptr(), wk.data_ptr(), wv.data_ptr(),
+        conv.data_ptr(), B, T, d, taps, dilation, eps, dh.data_ptr(), dk.data_ptr(), dv.data_ptr(), dw[0].data_ptr(),
+        dw[1].data_ptr(), dw[2].data_ptr(), dconv.data_ptr(), parts.data_ptr(), _stream(h))
+    _lib.check(rc, "smlm_engram_mix_backward")
+    return dh, dk, dv, dw[0], dw[1], dw[2], dconv

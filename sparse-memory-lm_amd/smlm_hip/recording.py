@@ -1,0 +1,24 @@
+"""When a kernel may stand in for a sequence of PyTorch ops that other machinery could be watching."""
+import torch
+from torch.autograd import forward_ad
+
+
+def ordinary(*tensors):
+    """Whether nothing but eager execution and reverse-mode recording sees these tensors: plain tensors, and no
+    compilation, tracing, function transform (vmap, grad, jvp), forward-mode level or dispatch mode is active.  Else the
+    PyTorch ops run, which all of these follow."""
+    return (all(t is None or type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and not torch._C._are_functorch_transforms_active() and forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0)
+
+
+def unhooked(*modules):
+    """Whether these modules' calls do nothing but their forward (no hooks), so that a kernel may read their weights."""
+    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                   for m in modules)
+
+
+def records(*tensors):
+    """Whether autograd records an op on these tensors."""
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)

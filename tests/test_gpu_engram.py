@@ -138,3 +138,120 @@ def test_row_sparse_training_matches_fp64_autograd():
     ed = md.engram_layers()[0]
     (ed(h.to(DEV), rows) * G.to(DEV)).sum().backward()
     assert float((ed.values.weight.grad.double().cpu() - p["values"].grad).abs().max()) <= 1e-5 * scale
+
+
+# ---------------------------------------------------------------------------------------- gate and convolution kernel
+MIX_SHAPES = [(1, 1, 8, 4, 3), (2, 31, 64, 4, 3), (3, 32, 384, 4, 3), (1, 33, 384, 4, 3), (2, 70, 512, 4, 10), (2, 41, 120, 1, 1),
+              (2, 100, 72, 2, 32), (1, 8, 512, 3, 16)]
+
+
+def _mix_inputs(B, T, d, taps, dtype, seed=0):
+    g = torch.Generator().manual_seed(seed + T + d)
+    h, k, v = (torch.randn(B, T, d, generator=g) for _ in range(3))
+    w = [torch.rand(d, generator=g) + 0.5 for _ in range(3)] + [torch.randn(d, 1, taps, generator=g) * 0.4]
+    return ([h.to(DEV, dtype)] + [t.to(DEV, torch.bfloat16) for t in (k, v)] + [t.to(DEV, dtype) for t in w])
+
+
+def _mix64(h, k, v, wh, wk, wv, conv, dilation, eps, left=None):
+    """(y, u of left and sequence, sum of |tap x u|) in fp64 on the CPU."""
+    B, T, d = h.shape
+    a = torch.sigmoid((E.rms_norm(h, wh, eps) * E.rms_norm(k, wk, eps)).sum(-1, keepdim=True) / d ** 0.5)
+    past = (conv.shape[2] - 1) * dilation
+    full = torch.cat([h.new_zeros(B, past, d) if left is None else left, E.rms_norm(a * v, wv, eps)], 1)
+    mass = E.causal_depthwise_conv(full.abs(), conv.abs(), dilation, T)
+    return torch.nn.functional.silu(E.causal_depthwise_conv(full, conv, dilation, T)) + a * v, full, mass
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,T,d,taps,dilation", MIX_SHAPES)
+@pytest.mark.parametrize("cached", [False, True])
+def test_engram_mix_against_fp64(B, T, d, taps, dilation, cached, dtype):
+    """Per element: u is rounded to bf16 (8 bits: within 2^-8 of each tap's term, and silu's slope is below 1.1), the result to its
+    type, and the fp32 arithmetic between (1e-5 of the largest value, a few hundred roundings of sums over d)."""
+    note(f"engram mix B={B} T={T} d={d} taps={taps} dilation={dilation} cached={cached} {dtype}")
+    args = _mix_inputs(B, T, d, taps, dtype)
+    past = (taps - 1) * dilation
+    left = torch.randn(B, past, d).to(DEV, torch.bfloat16) if cached else None
+    y, tail = K.engram_mix(*args, dilation, 1e-5, left, keep_tail=True)
+    assert torch.equal(K.engram_mix(*args, dilation, 1e-5, left), y) and y.dtype == dtype
+    ref, full, mass = _mix64(*(t.double().cpu() for t in args), dilation, 1e-5,
+                             None if left is None else left.double().cpu())
+    bound = 1.1 * 2 ** -8 * mass + 1e-5 * ref.abs().max() + (2 ** -8 * ref.abs() if dtype == torch.bfloat16 else 0)
+    assert bool(((y.double().cpu() - ref).abs() <= bound).all())
+    want = full[:, full.shape[1] - past:] if past else full[:, :0]
+    assert tail.shape == want.shape
+    assert bool(((tail.double().cpu() - want).abs() <= 2 ** -8 * want.abs() + 1e-5).all())
+
+
+@pytest.mark.parametrize("B,T,d,taps,dilation", MIX_SHAPES)
+def test_engram_mix_gradient_against_fp64(B, T, d, taps, dilation):
+    """Through the recorded node: bf16 roundings of u, of the convolution's output gradient and of dk and dv, each within
+    2^-8 of its value and below 2^-9 in the mean, so 2^-7 of each gradient's norm; the same bits on every call; a gradient of the gradient."""
+    note(f"engram mix gradient B={B} T={T} d={d} taps={taps} dilation={dilation}")
+    from smlm_hip.engram import _Mix
+    args = [t.requires_grad_() for t in _mix_inputs(B, T, d, taps, torch.float32, 5)]
+    gy = torch.randn(B, T, d, generator=torch.Generator().manual_seed(9)).to(DEV)
+    ref_args = [t.detach().double().cpu().requires_grad_() for t in args]
+    ref = torch.autograd.grad(_mix64(*ref_args, dilation, 1e-5)[0], ref_args, gy.double().cpu())
+    got = torch.autograd.grad(_Mix.apply(*args, dilation, 1e-5), args, gy)
+    for name, a, b, x in zip(("h", "k", "v", "wh", "wk", "wv", "conv"), got, ref, args):
+        assert a.dtype == x.dtype and a.shape == x.shape
+        err = float((a.double().cpu() - b).norm() / b.norm())
+        assert err <= 2 ** -7, (name, err)
+    again = torch.autograd.grad(_Mix.apply(*args, dilation, 1e-5), args, gy)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+    first = torch.autograd.grad(_Mix.apply(*args, dilation, 1e-5), args[0], gy, create_graph=True)[0]
+    second = torch.autograd.grad(first.square().sum(), args[1])[0]
+    f64 = torch.autograd.grad(_mix64(*ref_args, dilation, 1e-5)[0], ref_args[0], gy.double().cpu(), create_graph=True)[0]
+    s64 = torch.autograd.grad(f64.square().sum(), ref_args[1])[0]
+    assert float((second.double().cpu() - s64).norm()) <= 2 ** -4 * float(s64.norm())   # twice through bf16 ops
+
+
+def test_engram_module_takes_the_kernel_or_the_ops():
+    """The module's forward with and without the kernel: the same numbers within bf16, its results' types and cache; hooks,
+    other autocast types, forward-mode and recorded bf16 weights keep the PyTorch ops."""
+    note("engram module routes")
+    torch.manual_seed(3)
+    m = EngramMemory(64, 16, 24, 53).to(DEV)
+    m.conv.weight.data.normal_(std=0.3)
+    h, rows = torch.randn(2, 40, 64, device=DEV), torch.randint(0, 53, (2, 40, 16), device=DEV)
+    calls = []
+    real = K.engram_mix
+    ops = EngramMemory.gated_value
+
+    def count(f, *a):
+        K.engram_mix = lambda *x, **kw: (calls.append(1), real(*x, **kw))[1]
+        try:
+            calls.clear()
+            return f(*a), len(calls)
+        finally:
+            K.engram_mix = real
+
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        (y, n), hook = count(m, h, rows), m.k_norm.register_forward_hook(lambda *a: None)
+        (z, n2) = count(m, h, rows)
+        hook.remove()
+    assert (n, n2) == (1, 0) and y.dtype == z.dtype and y.requires_grad and z.requires_grad
+    assert float((y - z).norm()) <= 2 ** -6 * float(z.norm())
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+        assert count(m, h, rows)[1] == 0
+    assert count(m, h, rows)[1] == 0                                        # fp32 without autocast
+    b = EngramMemory(64, 16, 24, 53).to(DEV)
+    b.load_state_dict(m.state_dict())
+    b = b.to(torch.bfloat16)
+    assert count(b, h.bfloat16(), rows)[1] == 0                             # its weights record
+    with torch.no_grad():
+        caches = {}, {}
+        outs = []
+        for cache, kernel in zip(caches, (True, False)):
+            hook = None if kernel else b.v_norm.register_forward_hook(lambda *a: None)
+            parts = [count(b, h[:, s:e].bfloat16(), rows[:, s:e], cache) for s, e in ((0, 3), (3, 4), (4, 40))]
+            assert [c for _, c in parts] == ([1] * 3 if kernel else [0] * 3)
+            outs.append(torch.cat([p for p, _ in parts], 1))
+            hook and hook.remove()
+        assert outs[0].dtype == outs[1].dtype
+        assert float((outs[0] - outs[1]).float().norm()) <= 2 ** -6 * float(outs[1].float().norm())
+        assert caches[0]["eng_u"].shape == caches[1]["eng_u"].shape and caches[0]["eng_u"].dtype == caches[1]["eng_u"].dtype
+        with torch.autograd.forward_ad.dual_level():
+            assert count(b, h.bfloat16(), rows)[1] == 0
+    assert EngramMemory.gated_value is ops
