@@ -40,23 +40,35 @@ struct MixGradArgs {
   float *parts;     // (workgroups, (3 + taps) d): dwh, dwk, dwv, then each tap's dconv
 };
 
-// 8 adjacent values as fp32, zeros past the width.
+// 8 adjacent values as they lie in memory, zeros past the width, and as fp32.
+template <bool F32>
+struct Raw8 {
+  uint4 a[F32 ? 2 : 1];
+};
+template <bool F32>
+__device__ __forceinline__ Raw8<F32> raw8(const void *p, int64_t o, bool in) {
+  Raw8<F32> r = {};
+  if (in) {
+    r.a[0] = *(const uint4 *)((const char *)p + o * (F32 ? 4 : 2));
+    if constexpr (F32) r.a[1] = *(const uint4 *)((const char *)p + o * 4 + 16);
+  }
+  return r;
+}
+template <bool F32>
+__device__ __forceinline__ void unpack8(const Raw8<F32> &r, float *x) {
+#pragma unroll
+  for (int i = 0; i < (F32 ? 2 : 1); ++i) {
+    const uint32_t t[4] = {r.a[i].x, r.a[i].y, r.a[i].z, r.a[i].w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (F32) x[4 * i + e] = __uint_as_float(t[e]);
+      else x[2 * e] = __uint_as_float(t[e] << 16), x[2 * e + 1] = __uint_as_float(t[e] & 0xFFFF0000u);
+    }
+  }
+}
 template <bool F32>
 __device__ __forceinline__ void load8(const void *p, int64_t o, bool in, float *x) {
-  if constexpr (F32) {
-    float4 a = {}, b = {};
-    if (in) {
-      a = *(const float4 *)((const float *)p + o);
-      b = *(const float4 *)((const float *)p + o + 4);
-    }
-    x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w, x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
-  } else {
-    uint4 a = {};
-    if (in) a = *(const uint4 *)((const uint16_t *)p + o);
-    const uint32_t t[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) x[2 * i] = bf16_bits_to_f32(t[i] & 0xFFFFu), x[2 * i + 1] = bf16_bits_to_f32(t[i] >> 16);
-  }
+  unpack8<F32>(raw8<F32>(p, o, in), x);
 }
 template <bool F32>
 __device__ __forceinline__ void store8(void *p, int64_t o, const float *x) {
@@ -93,6 +105,19 @@ __device__ __forceinline__ void load_weights(const MixArgs &A, int col, bool in,
   load8<HF32>(A.wh, col, in, W.h);
   load8<HF32>(A.wk, col, in, W.k);
   load8<HF32>(A.wv, col, in, W.v);
+}
+template <bool HF32>
+__device__ __forceinline__ void load_taps(const MixArgs &A, int col, bool in, MixWeights &W) {
+  if (A.taps == kMixTaps && (uintptr_t)A.conv % 16 == 0) {  // the lane's 8 x 4 taps are adjacent
+    float x[8 * kMixTaps];
+#pragma unroll
+    for (int i = 0; i < kMixTaps; ++i) load8<HF32>(A.conv, (int64_t)col * kMixTaps + 8 * i, in, x + 8 * i);
+#pragma unroll
+    for (int i = 0; i < kMixTaps; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) W.conv[i][e] = x[e * kMixTaps + i];
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < kMixTaps; ++i)
 #pragma unroll
@@ -127,10 +152,23 @@ __device__ __forceinline__ void mix_sums(const MixToken &t, const MixWeights &W,
   }
 }
 template <bool HF32>
+struct RawToken {
+  Raw8<HF32> h;
+  Raw8<false> k, v;
+};
+template <bool HF32>
+__device__ __forceinline__ RawToken<HF32> raw_token(const MixArgs &A, int64_t o, bool in) {
+  return {raw8<HF32>(A.h, o, in), raw8<false>(A.k, o, in), raw8<false>(A.v, o, in)};
+}
+template <bool HF32>
+__device__ __forceinline__ void unpack_token(const RawToken<HF32> &r, MixToken &t) {
+  unpack8<HF32>(r.h, t.h);
+  unpack8<false>(r.k, t.k);
+  unpack8<false>(r.v, t.v);
+}
+template <bool HF32>
 __device__ __forceinline__ void load_token(const MixArgs &A, int64_t o, bool in, MixToken &t) {
-  load8<HF32>(A.h, o, in, t.h);
-  load8<false>(A.k, o, in, t.k);
-  load8<false>(A.v, o, in, t.v);
+  unpack_token<HF32>(raw_token<HF32>(A, o, in), t);
 }
 __device__ __forceinline__ void token_u(const MixArgs &A, const MixWeights &W, MixToken &t, float *gv, float *u) {
   float s[4];
@@ -166,11 +204,11 @@ __global__ void __launch_bounds__(kMixThreads) engram_mix_kernel(MixArgs A) {
   const int64_t b = blockIdx.x / A.tiles;
   const int t0 = (int)(blockIdx.x % A.tiles) * kMixTokens;
   const int64_t base = b * A.T * A.d + col, side = b * past * A.d + col;
-  MixToken tok[kMixPer];
+  RawToken<HF32> tok[kMixPer];
 #pragma unroll
   for (int j = 0; j < kMixPer; ++j) {  // the tile's loads first; tokens past the end read the last one
     const int t = min(t0 + wave + j * kMixWaves, A.T - 1);
-    load_token<HF32>(A, base + (int64_t)t * A.d, in, tok[j]);
+    tok[j] = raw_token<HF32>(A, base + (int64_t)t * A.d, in);
   }
   MixWeights W;
   load_weights<HF32>(A, col, in, W);
@@ -179,7 +217,9 @@ __global__ void __launch_bounds__(kMixThreads) engram_mix_kernel(MixArgs A) {
   for (int j = 0; j < kMixPer; ++j) {
     const int q = wave + j * kMixWaves, t = t0 + q;
     float u[8];
-    token_u(A, W, tok[j], gv[j], u);
+    MixToken x;
+    unpack_token<HF32>(tok[j], x);
+    token_u(A, W, x, gv[j], u);
     if (in) store8<false>(u_rows, (int64_t)(past + q) * A.d + col, u);
     if (A.tail && in && t < A.T && t >= A.T - past) store8<false>(A.tail, side + (int64_t)(t - (A.T - past)) * A.d, u);
   }
@@ -203,6 +243,7 @@ __global__ void __launch_bounds__(kMixThreads) engram_mix_kernel(MixArgs A) {
       if (in) store8<false>(A.tail, side + (int64_t)i * A.d, u);
     }
   }
+  load_taps<HF32>(A, col, in, W);
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < kMixPer; ++j) {
@@ -232,6 +273,7 @@ __global__ void __launch_bounds__(kMixThreads) engram_mix_backward_kernel(MixArg
   uint16_t *dc_rows = lds + (kMixTokens + 2 * past) * A.d;      // (32 + past, d): row q is token t0 + q
   MixWeights W;
   load_weights<true>(A, col, in, W);
+  load_taps<true>(A, col, in, W);
   for (int i = wave; i < kMixTokens + 2 * past; i += kMixWaves) {
     const int t = t0 - past + i;
     float u[8] = {}, g[8];
