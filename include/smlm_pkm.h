@@ -268,6 +268,24 @@ int smlm_prefill_attention(const void *q, const int64_t *q_strides, const void *
                            int H, int T, int S, int head_dim, void *stream);
 
 /*
+ * Training form of causal self-attention (S == T) on q, k after RoPE, and its gradient.
+ * smlm_attention_train: smlm_prefill_attention for q, k (B, H, T, head_dim) contiguous and v, y with strides over
+ * (b, h, t), which also writes lse[(b H + h) lse_stride + t] = log2 sum_s exp(score) in fp32.
+ * smlm_attention_backward: from dy (strides of y) the gradient dqkv (B, T, 3, H, head_dim) bf16 contiguous of the qkv
+ * projection whose RoPE (rope_cos, rope_sin (rope_len, head_dim / 2), positions pos0 + t) gave q and k.  Probabilities
+ * recomputed from q, k and lse; fp32 scores, probabilities and sums, bf16 operands of the products.  lse and delta
+ * (scratch) (B H, row_stride) fp32 with row_stride a multiple of 64, at least T.  Two launches, no atomics: the same
+ * result on every call.  head_dim in {32, 64, 128}; tensors 16-byte aligned, strides multiples of 8 elements.
+ */
+int smlm_attention_train(const void *q, const void *k, const void *v, const int64_t *v_strides, void *y,
+                         const int64_t *y_strides, float *lse, int64_t lse_stride, int64_t B, int H, int T, int head_dim,
+                         void *stream);
+int smlm_attention_backward(const void *q, const void *k, const void *v, const int64_t *v_strides, const void *y,
+                            const void *dy, const int64_t *y_strides, const float *lse, float *delta,
+                            int64_t row_stride, const void *rope_cos, const void *rope_sin, int rope_dtype,
+                            int rope_len, int pos0, void *dqkv, int64_t B, int H, int T, int head_dim, void *stream);
+
+/*
  * Fused linear layer of the single-token decode step (M = decode batch rows):  y = h W^T on the matrix cores with
  * the op in front of it and the op after it in one launch.  Replaces, per decode step, the nn.Linear calls of
  * smlm/model.py:90-118 and 266-293 (wqkv, wo, w13, w2, lm_head) and smlm/pkm.py:188-191, 213-224 (query_proj,

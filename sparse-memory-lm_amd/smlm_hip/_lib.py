@@ -58,6 +58,8 @@ EXPORTS = {
     "smlm_affine_bf16": (_i, [_p, _i64, _p, _p, _i64, _i, _p, _i64, _p]),
     "smlm_rope_qkv": (_i, [_p, _i64, _p, _p, _i, _i, _i, _p, _p, _p, _p, _p, _p, _i64, _i, _i, _i, _p]),
     "smlm_prefill_attention": (_i, [_p, _p, _p, _p, _p, _p, _p, _p, _i64, _i, _i, _i, _i, _p]),
+    "smlm_attention_train": (_i, [_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i, _i, _i, _p]),
+    "smlm_attention_backward": (_i, [_p] * 9 + [_i64, _p, _p, _i, _i, _i, _p, _i64, _i, _i, _i, _p]),
     "smlm_linear_argmax_blocks": (_i, [_i]),
     "smlm_decode_linear": (_i, [ctypes.POINTER(LinearArgs), _p]),
     "smlm_argmax_finish": (_i, [_p, _i64, _i, _i64, _p, _p, _p, _i64, _i64, _i, _p]),

@@ -417,6 +417,58 @@ def prefill_attention(q, k, v, out=None):
     return out
 
 
+def _v_of(qkv, H):
+    """The values' (B, T, H, hd) view of a contiguous qkv projection (B, T, 3*H*hd)."""
+    B, T, C3 = qkv.shape
+    return qkv.view(B, T, 3, H, C3 // (3 * H))[:, :, 2]
+
+
+def attention_train(qkv, rope_cos, rope_sin, pos0, H):
+    """Causal self-attention of a qkv projection (B, T, 3*H*hd) bf16, hd in (32, 64, 128), with what its gradient needs:
+    RoPE at positions pos0 .. (rope_qkv) and prefill_attention, returning (y (B, T, H*hd) bf16, q and k after RoPE
+    (B, H, T, hd), lse (B*H, T rounded up to 64) fp32)."""
+    _need_cuda("attention_train", qkv)
+    qkv = qkv.contiguous()
+    B, T, C3 = qkv.shape
+    hd = C3 // (3 * H)
+    if C3 != 3 * H * hd or hd not in (32, 64, 128):
+        raise ValueError(f"attention_train: qkv {tuple(qkv.shape)} with {H} heads: head_dim must be 32, 64 or 128")
+    q = torch.empty(B, H, T, hd, dtype=torch.bfloat16, device=qkv.device)
+    k = torch.empty_like(q)
+    rope_qkv(qkv, rope_cos, rope_sin, pos0, q, k)
+    v = _v_of(qkv, H)
+    y = torch.empty(B, T, H * hd, dtype=torch.bfloat16, device=qkv.device)
+    lse = torch.empty(B * H, -(-T // 64) * 64, dtype=torch.float32, device=qkv.device)
+    vs = (ctypes.c_int64 * 3)(v.stride(0), v.stride(2), v.stride(1))
+    ys = (ctypes.c_int64 * 3)(T * H * hd, hd, H * hd)
+    rc = _lib.lib().smlm_attention_train(q.data_ptr(), k.data_ptr(), v.data_ptr(), vs, y.data_ptr(), ys, lse.data_ptr(),
+                                         lse.stride(0), B, H, T, hd, _stream(qkv))
+    _lib.check(rc, "smlm_attention_train")
+    return y, q, k, lse
+
+
+def attention_backward(dy, qkv, y, q, k, lse, rope_cos, rope_sin, pos0):
+    """The gradient (B, T, 3*H*hd) bf16 of attention_train's qkv from dy (B, T, H*hd) bf16 and what it returned
+    (smlm_attention_backward).  The same result on every call."""
+    _need_cuda("attention_backward", dy, qkv, y, q, k, lse, rope_cos, rope_sin)
+    B, H, T, hd = q.shape
+    if dy.dtype != torch.bfloat16 or tuple(dy.shape) != (B, T, H * hd) or tuple(qkv.shape) != (B, T, 3 * H * hd):
+        raise ValueError(f"attention_backward: dy must be ({B}, {T}, {H * hd}) bf16")
+    if rope_cos.dtype not in _DT or rope_sin.dtype != rope_cos.dtype or rope_cos.shape != rope_sin.shape \
+            or rope_cos.dim() != 2 or rope_cos.shape[1] != hd // 2:
+        raise ValueError("attention_backward: rope tables must be (max_seq_len, head_dim/2) fp32 or bf16")
+    qkv, dy, rope_cos, rope_sin = qkv.contiguous(), _aligned(dy), rope_cos.contiguous(), rope_sin.contiguous()
+    v, dqkv, delta = _v_of(qkv, H), torch.empty_like(qkv), torch.empty_like(lse)
+    vs = (ctypes.c_int64 * 3)(v.stride(0), v.stride(2), v.stride(1))
+    ys = (ctypes.c_int64 * 3)(T * H * hd, hd, H * hd)
+    rc = _lib.lib().smlm_attention_backward(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), vs, y.data_ptr(), dy.data_ptr(), ys, lse.data_ptr(), delta.data_ptr(),
+        lse.stride(0), rope_cos.data_ptr(), rope_sin.data_ptr(), _DT[rope_cos.dtype], rope_cos.shape[0], pos0,
+        dqkv.data_ptr(), B, H, T, hd, _stream(qkv))
+    _lib.check(rc, "smlm_attention_backward")
+    return dqkv
+
+
 def swiglu(h13):
     """h13 (..., 2*hidden) bf16, the w13 projection -> (..., hidden) bf16 = bf16(bf16(silu(a)) * b) with a, b its
     two halves (smlm/model.py:110-118)."""

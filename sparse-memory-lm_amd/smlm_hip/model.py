@@ -18,6 +18,7 @@ from torch import nn
 from . import kernels
 from .engram import EngramMemory, NgramHash
 from .pkm import ProductKeyMemory, inference_tables, state_tag, state_tensors
+from .recording import ordinary, records, unhooked
 
 
 @dataclass
@@ -128,6 +129,8 @@ class Attention(nn.Module):
         qkv = kernels.linear(self.wqkv, x)
         if not torch.is_tensor(pos0) and _use_attention_kernels(qkv, self.head_dim):
             return kernels.linear(self.wo, self._prefill_kernels(qkv, kv_cache, pos0).reshape(B, T, C))
+        if kv_cache is None and not torch.is_tensor(pos0) and self._train_kernels(qkv, pos0):
+            return self.wo(_AttentionTrain.apply(qkv, self.rope, pos0, self.n_heads))
         q, k, v = qkv.view(B, T, 3, self.n_heads, self.head_dim).permute(2, 0, 3, 1, 4)
         q, k = self.rope(q, pos0), self.rope(k, pos0)
         if isinstance(kv_cache, StaticKVCache):
@@ -140,6 +143,17 @@ class Attention(nn.Module):
                 kv_cache["k"], kv_cache["v"] = k, v
             y = _causal_attention(q, k, v)
         return kernels.linear(self.wo, y.reshape(B, T, C))
+
+    def _train_kernels(self, qkv, pos0):
+        """Whether a recorded pass over a whole sequence runs as one node on the kernels: bf16 on the GPU (bf16 weights
+        or autocast), plain reverse-mode recording (ordinary), positions inside the rope table."""
+        rope = self.rope
+        cos, sin = rope.cos, rope.sin
+        return (qkv.is_cuda and qkv.dtype == torch.bfloat16 and self.head_dim in (32, 64, 128) and qkv.numel() > 0
+                and records(qkv) and type(rope) is RotaryEmbedding and unhooked(rope)
+                and cos.dtype in (torch.float32, torch.bfloat16) and sin.dtype == cos.dtype and not records(cos, sin)
+                and cos.device == sin.device == qkv.device and 0 <= pos0 and pos0 + qkv.shape[1] <= cos.shape[0]
+                and ordinary(qkv, cos, sin))
 
     def _prefill_kernels(self, qkv, kv_cache, pos0):
         """RoPE (smlm_rope_qkv, written straight into the static cache's slots when there is one) and causal
@@ -177,6 +191,30 @@ class Attention(nn.Module):
         cache.v[:, :, pos0:pos0 + T] = v
         S = pos0 + T
         return _causal_attention(q, cache.k[:, :, :S], cache.v[:, :, :S])
+
+
+class _AttentionTrain(torch.autograd.Function):
+    """RoPE and causal self-attention of a qkv projection (B, T, 3 C) bf16, recorded as one node: forward and gradient
+    on the matrix cores without a (T, T) tensor (kernels.attention_train, attention_backward).  A backward that is
+    itself recorded (create_graph) differentiates the PyTorch ops."""
+
+    @staticmethod
+    def forward(ctx, qkv, rope, pos0, n_heads):
+        y, q, k, lse = kernels.attention_train(qkv, rope.cos, rope.sin, pos0, n_heads)
+        ctx.save_for_backward(qkv, y, q, k, lse, rope.cos, rope.sin)
+        ctx.rope, ctx.pos0, ctx.n_heads = rope, pos0, n_heads
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        qkv, *saved, cos, sin = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            B, T, C3 = qkv.shape
+            q, k, v = qkv.view(B, T, 3, ctx.n_heads, -1).permute(2, 0, 3, 1, 4)
+            q, k = ctx.rope(q, ctx.pos0), ctx.rope(k, ctx.pos0)
+            y = _attention(q, k, v, _causal_mask(T, T, q.device)).transpose(1, 2).reshape(B, T, C3 // 3)
+            return torch.autograd.grad(y, qkv, dy, create_graph=True)[0], None, None, None
+        return kernels.attention_backward(dy, qkv, *saved, cos, sin, ctx.pos0), None, None, None
 
 
 def _causal_mask(T, S, device):

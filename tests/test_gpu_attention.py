@@ -384,3 +384,97 @@ def test_prompt_linear_affine_equals_the_two_launches(M):
     assert float((fused.float() != ref).double().mean()) <= 1e-3
     with pytest.raises(ValueError):
         K.prompt_linear(x, w, b, scale, None)
+
+
+# ------------------------------------------------------------------------------------------------ training
+def _attention64(qkv, cos, sin, pos0, H):
+    """RoPE and causal attention of qkv (B, T, 3 C) in its own precision, (B, T, C)."""
+    B, T, C3 = qkv.shape
+    q, k, v = qkv.view(B, T, 3, H, -1).permute(2, 0, 3, 1, 4)
+    c, s = cos[pos0:pos0 + T], sin[pos0:pos0 + T]
+    rope = lambda u: torch.cat([u.chunk(2, -1)[0] * c - u.chunk(2, -1)[1] * s,  # noqa: E731
+                                u.chunk(2, -1)[0] * s + u.chunk(2, -1)[1] * c], -1)
+    q, k = rope(q), rope(k)
+    p = (q @ k.transpose(-1, -2)) / q.shape[-1] ** 0.5
+    p = torch.softmax(p.masked_fill(~torch.ones(T, T, dtype=torch.bool).tril(), float("-inf")), -1)
+    return (p @ v).transpose(1, 2).reshape(B, T, C3 // 3)
+
+
+@pytest.mark.parametrize("rope_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,H,T,hd,pos0", [(1, 1, 1, 32, 0), (2, 3, 2, 64, 5), (1, 2, 63, 128, 0), (2, 1, 64, 32, 3),
+                                           (1, 3, 65, 64, 0), (1, 2, 127, 64, 0), (1, 1, 129, 128, 7), (2, 2, 200, 32, 0),
+                                           (1, 6, 321, 64, 0), (1, 2, 450, 128, 0)])
+def test_attention_gradient_against_fp64(B, H, T, hd, pos0, rope_dtype):
+    """The recorded node against fp64 autograd on the CPU.  Roundings to bf16 within 2^-8 each, below 2^-9 in the mean: q
+    and k after RoPE, P and dS as operands, y in delta, and the gradient itself: 2^-6 of each gradient's norm.  The same
+    bits on every call."""
+    print(f"attention gradient B={B} H={H} T={T} hd={hd} pos0={pos0} {rope_dtype}", flush=True)
+    from smlm_hip.model import RotaryEmbedding, _AttentionTrain
+    g = torch.Generator().manual_seed(T + hd)
+    rope = RotaryEmbedding(hd, pos0 + T, 10000.0).to(DEV, rope_dtype)
+    qkv = torch.randn(B, T, 3 * H * hd, generator=g).to(DEV, torch.bfloat16).requires_grad_()
+    dy = torch.randn(B, T, H * hd, generator=g).to(DEV, torch.bfloat16)
+    y = _AttentionTrain.apply(qkv, rope, pos0, H)
+    got = torch.autograd.grad(y, qkv, dy, retain_graph=True)[0]
+    assert got.dtype == torch.bfloat16
+    assert torch.equal(torch.autograd.grad(_AttentionTrain.apply(qkv, rope, pos0, H), qkv, dy)[0], got)
+    x = qkv.detach().double().cpu().requires_grad_()
+    ref_y = _attention64(x, rope.cos.double().cpu(), rope.sin.double().cpu(), pos0, H)
+    ref = torch.autograd.grad(ref_y, x, dy.double().cpu())[0]
+    assert float((y.double().cpu() - ref_y).detach().norm()) <= 2 ** -7 * float(ref_y.detach().norm())
+    for part, name in enumerate("qkv"):
+        a, b = (t.double().cpu().view(B, T, 3, -1)[:, :, part] for t in (got, ref))
+        whole = float(ref.norm()) / 3                       # a sequence of one or two tokens has no dq and dk to speak of
+        assert float((a - b).norm()) <= 2 ** -6 * max(float(b.norm()), whole), name
+        assert not torch.isnan(a).any()
+
+
+def test_attention_training_routes():
+    """The attention block under bf16 autocast: the kernels' results agree with the PyTorch ops' within bf16, a gradient
+    of the gradient exists, and hooks, forward-mode, dispatch modes, caches and fp32 keep the ops."""
+    print("attention training routes", flush=True)
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from smlm_hip.model import Attention, ModelConfig
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    torch.manual_seed(0)
+    a = Attention(ModelConfig(d_model=128, n_heads=2, max_seq_len=100)).to(DEV)
+    x = torch.randn(2, 100, 128, device=DEV, requires_grad=True)
+    used = []
+    real = K.attention_train
+
+    def run(**kw):
+        K.attention_train = lambda *p: (used.append(1), real(*p))[1]
+        used.clear()
+        try:
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                return a(x, **kw), len(used)
+        finally:
+            K.attention_train = real
+
+    y, n = run()
+    hook = a.rope.register_forward_hook(lambda *p: None)
+    z, n2 = run()
+    assert (n, n2) == (1, 0) and y.dtype == z.dtype
+    gy, gz = (torch.autograd.grad(t.float().square().sum(), [x, a.wqkv.weight, a.wo.weight]) for t in (y, z))
+    for p, q in zip((y, *gy), (z, *gz)):
+        assert p.dtype == q.dtype and float((p - q).detach().float().norm()) <= 2 ** -5 * float(q.detach().float().norm())
+    second = []
+    for keep in (True, False):                              # with the hook: the ops
+        t, n = run()
+        assert n == (0 if keep else 1)
+        dx = torch.autograd.grad(t.float().square().sum(), x, create_graph=True)[0]
+        second.append(torch.autograd.grad(dx.square().sum(), a.wqkv.weight)[0])
+        if keep:
+            hook.remove()
+    assert float((second[0] - second[1]).norm()) <= 2 ** -4 * float(second[0].norm())
+    with Watch():
+        assert run()[1] == 0
+    with torch.autograd.forward_ad.dual_level():
+        assert run()[1] == 0
+    assert run(kv_cache={})[1] == 0
+    assert a(x).dtype == torch.float32 and not used[1:]
