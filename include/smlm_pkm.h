@@ -402,6 +402,17 @@ int smlm_pkm_select_backward(const int64_t *idx, const float *w, const void *g_s
                              int64_t N, int H, int NK, int knn, void *ds1, void *ds2, void *stream);
 
 /*
+ * Gradient of the memory query's batch normalisation in training (smlm/pkm.py:188-191), y = (x - mean) invstd weight +
+ * bias over N rows: from g and x (N, C) bf16 contiguous and the forward's mean, invstd (C,) fp32, dx (N, C) bf16, dweight
+ * and dbias (C,) fp32.  parts: caller-owned scratch of smlm_query_norm_parts(N, C) doubles; k: of 2 C floats.  N >= 2, C
+ * a multiple of 8; g, x, dx, parts 16-byte aligned.  Sums in 64 bits in a fixed order.
+ */
+int64_t smlm_query_norm_parts(int64_t N, int C);
+int smlm_query_norm_backward(const void *g, const void *x, const float *weight, const float *mean, const float *invstd,
+                             int64_t N, int C, double *parts, float *k, void *dx, float *dweight, float *dbias,
+                             void *stream);
+
+/*
  * Row-sparse value-bag backward (smlm/kernels.py:1-104, smlm/sparse_values.py:94-113):
  *   acc[idx[n,k], :] += w[n,k] * grad_out[n, :]   (fp32 atomic adds: the order of additions is not fixed)
  *   touched[idx[n,k]] = 1

@@ -837,6 +837,27 @@ class PKSelect(torch.autograd.Function):
         return ds1, ds2, None
 
 
+def query_norm_backward(g, x, weight, mean, invstd):
+    """Gradient of the memory query's batch norm in training (smlm/pkm.py:188-191) from g and x (N >= 2, C) bf16, weight
+    and the forward's mean and 1 / sqrt(var + eps) (C,) fp32: (dx (N, C) bf16, dweight, dbias (C,) fp32).  C a multiple
+    of 8."""
+    _need_cuda("query_norm_backward", g, x, weight, mean, invstd)
+    if x.dtype != torch.bfloat16 or x.dim() != 2 or g.dtype != x.dtype or g.shape != x.shape:
+        raise ValueError(f"query_norm_backward: g and x must be (N, C) bf16, got {tuple(g.shape)} and {tuple(x.shape)}")
+    N, C = x.shape
+    if any(t.dtype != torch.float32 or t.shape != (C,) for t in (weight, mean, invstd)):
+        raise ValueError(f"query_norm_backward: weight and statistics must be ({C},) fp32")
+    x, g, weight, mean, invstd = _aligned(x), _aligned(g), weight.contiguous(), mean.contiguous(), invstd.contiguous()
+    L = _lib.lib()
+    parts = torch.empty(L.smlm_query_norm_parts(N, C), dtype=torch.float64, device=x.device)
+    cols, dx = torch.empty(4, C, dtype=torch.float32, device=x.device), torch.empty_like(x)
+    rc = L.smlm_query_norm_backward(g.data_ptr(), x.data_ptr(), weight.data_ptr(), mean.data_ptr(), invstd.data_ptr(),
+                                    N, C, parts.data_ptr(), cols[2].data_ptr(), dx.data_ptr(), cols[0].data_ptr(),
+                                    cols[1].data_ptr(), _stream(x))
+    _lib.check(rc, "smlm_query_norm_backward")
+    return dx, cols[0], cols[1]
+
+
 def bag_backward_rows(grad_out, indices, weights, table, acc, touched, ordered=True, weight_grad=True):
     """Row-sparse bag backward (smlm/kernels.py:90-104): acc[indices[n, k]] += weights[n, k] * grad_out[n] and
     touched[indices] = True, in place; returns the per-sample-weight gradient (N, K) fp32.  table fp32 / bf16

@@ -25,6 +25,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from . import kernels
+from .recording import ordinary, records, unhooked
 from .sparse_values import check_impl, row_sparse_embedding_bag
 
 
@@ -34,6 +35,33 @@ def _pow2(n):
 
 def _autocast_bf16(x):
     return x.is_cuda and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
+
+
+class _QueryNorm(torch.autograd.Function):
+    """bf16(BatchNorm(q)) in training for a bf16 projection, recorded as one node: torch's batch norm on the fp32 copy
+    between the two casts, and its gradient from the bf16 tensors as they are (kernels.query_norm_backward).  A backward
+    that is itself recorded (create_graph) differentiates the PyTorch ops."""
+
+    @staticmethod
+    def forward(ctx, q, weight, bias, running_mean, running_var, momentum, eps):
+        y, mean, invstd = torch.native_batch_norm(q.float(), weight, bias, running_mean, running_var, True, momentum, eps)
+        ctx.save_for_backward(q, weight, bias, mean, invstd)
+        ctx.eps = eps
+        return y.to(q.dtype)
+
+    @staticmethod
+    def backward(ctx, g):
+        q, weight, bias, mean, invstd = ctx.saved_tensors
+        need = ctx.needs_input_grad[:3]
+        if torch.is_grad_enabled():
+            y = F.batch_norm(q.float(), None, None, weight, bias, True, 0.0, ctx.eps).to(q.dtype)
+            wanted = [t for t, n in zip((q, weight, bias), need) if n]
+            grads = iter(torch.autograd.grad(y, wanted, g, create_graph=True))
+            grads = [next(grads) if n else None for n in need]
+        else:
+            grads = [t if n else None
+                     for t, n in zip(kernels.query_norm_backward(g, q, weight, mean, invstd), need)]
+        return (*grads, None, None, None, None)
 
 
 def inference_tables(values):
@@ -262,13 +290,34 @@ class ProductKeyMemory(nn.Module):
             self._bn_cache = (tag, scale, shift)
         return self._bn_cache[1], self._bn_cache[2]
 
+    def _train_norm(self, q, to_bf16):
+        """The query's BatchNorm in training: fp32 whatever autocast does; a bf16 projection whose result goes on in
+        bf16 has its gradient on the kernel (_QueryNorm)."""
+        bn = self.query_norm
+        stats = (bn.running_mean, bn.running_var) if bn.track_running_stats else (None, None)
+        columns = (bn.weight, bn.bias, *stats)
+        if (to_bf16 and type(bn) is nn.BatchNorm1d and bn.training and q.is_cuda and q.dtype == torch.bfloat16
+                and q.dim() == 2 and q.shape[0] > 1 and q.shape[1] % 8 == 0 and bn.affine and bn.momentum is not None
+                and unhooked(bn) and records(q, bn.weight, bn.bias) and not records(*stats)
+                and all(t is None or (t.dtype == torch.float32 and t.device == q.device and t.is_contiguous()
+                                      and t.shape == (q.shape[1],)) for t in columns)
+                and (stats[0] is None) == (stats[1] is None) and ordinary(q, *columns)):
+            if bn.track_running_stats and bn.num_batches_tracked is not None:
+                bn.num_batches_tracked.add_(1)
+            if stats[0] is not None:
+                # torch's batch norm writes the statistics without a new version, by which _bn_affine and the captured
+                # graphs know that they changed
+                torch.autograd.graph.increment_version(stats)
+            return _QueryNorm.apply(q, *columns, bn.momentum, bn.eps)
+        return bn(q.to(bn.weight.dtype))
+
     def _train_forward(self, x):
         """The differentiable lookup (smlm/pkm.py:186-228 with impl="triton"): the kernels' selection with its
         backward (kernels.PKSelect), row-sparse or dense value gradients."""
         N = x.shape[0]
         q = self.query_proj(x)
         if self.query_norm is not None:
-            q = self.query_norm(q.to(self.query_norm.weight.dtype))     # BN in fp32 under autocast
+            q = self._train_norm(q, _autocast_bf16(x))
         q = q.view(N, self.heads, self.k_dim)
         if _autocast_bf16(x):
             q = q.to(torch.bfloat16)

@@ -499,3 +499,86 @@ def test_layer_training_step_matches_fp64_autograd(value_grad, score_scale):
     np.testing.assert_array_equal(table.detach().cpu().numpy(), p1)
     np.testing.assert_array_equal(opt.state[table]["exp_avg"].cpu().numpy(), m1)
     assert not st.touched.any() and not st.acc.any()
+
+
+# ---------------------------------------------------------------------------------------- the query's batch norm
+@pytest.mark.parametrize("N,C,shift", [(2, 8, 0.0), (31, 24, 3.0), (33, 264, 0.0), (257, 512, 40.0), (1000, 2048, 1.0),
+                                       (4099, 256, 0.0), (20000, 8, 5.0)])
+def test_query_norm_against_fp64(N, C, shift):
+    """The recorded node's result, running statistics, gradient and gradient's gradient against fp64 torch: the results within their
+    bf16 rounding (2^-8) and the fp32 arithmetic's (1e-5 of the largest value; times shift, for the cancellation of
+    x - mean), the running statistics
+    (fp32 sums) and the weights' gradients (64-bit sums of fp32 terms) within 1e-5."""
+    note(f"query norm N={N} C={C} shift={shift}")
+    from smlm_hip.pkm import _QueryNorm
+    g = torch.Generator().manual_seed(N + C)
+    x = (torch.randn(N, C, generator=g) + shift * torch.randn(C, generator=g)).to(torch.bfloat16)
+    w, b = torch.rand(C, generator=g) + 0.5, torch.randn(C, generator=g)
+    gy = torch.randn(N, C, generator=g).to(torch.bfloat16)
+    rm, rv = torch.randn(C, generator=g), torch.rand(C, generator=g) + 0.5
+    ref_in = [t.double().requires_grad_() for t in (x, w, b)]
+    rms = [rm.double(), rv.double()]
+    ref = torch.nn.functional.batch_norm(ref_in[0], *rms, *ref_in[1:], True, 0.1, 1e-5)
+    ref_g = torch.autograd.grad(ref, ref_in, gy.double(), create_graph=True)
+    ins = [t.to(DEV).requires_grad_() for t in (x, w, b)]
+    stats = [rm.to(DEV), rv.to(DEV)]
+    y = _QueryNorm.apply(*ins, *stats, 0.1, 1e-5)
+    slack = 1e-5 * (1 + shift)
+    for got, want in zip((y, *stats), (ref.detach(), *rms)):
+        tol = (2 ** -8 if got.dtype == torch.bfloat16 else 1e-5) * want.abs() + slack * want.abs().max()
+        assert bool(((got.detach().double().cpu() - want).abs() <= tol).all())
+    got_g = torch.autograd.grad(y, ins, gy.to(DEV), retain_graph=True)
+    for got, want, t in zip(got_g, ref_g, ins):
+        assert got.dtype == t.dtype
+        tol = (2 ** -8 * want.abs() if t is ins[0] else 0) + 10 * slack * want.abs().max()
+        if N > 2:                     # two rows: the gradient is a difference of equal numbers
+            assert bool(((got.double().cpu() - want).abs() <= tol).all())
+    again = torch.autograd.grad(_QueryNorm.apply(*ins, None, None, 0.1, 1e-5), ins, gy.to(DEV))
+    assert all(torch.equal(a, c) for a, c in zip(again, got_g))
+    if N > 2:
+        first = torch.autograd.grad(y, ins, gy.to(DEV), create_graph=True)
+        second = torch.autograd.grad(first[1].square().sum(), ins[0])[0].double().cpu()
+        want = torch.autograd.grad(ref_g[1].square().sum(), ref_in[0])[0]
+        assert float((second - want).norm()) <= 2 ** -6 * float(want.norm())
+
+
+def test_query_norm_routes():
+    """The training forward takes the kernel for a bf16 query under bf16 autocast; eval statistics, hooks, one row and
+    fp32 keep nn.BatchNorm1d, with the same results, running statistics and batch count."""
+    note("query norm routes")
+    from smlm_hip.pkm import ProductKeyMemory
+    torch.manual_seed(0)
+    ms = [ProductKeyMemory(64, 64, n_keys=32, heads=2, knn=8, k_dim=32, value_grad="row_sparse").to(DEV) for _ in range(2)]
+    ms[1].load_state_dict(ms[0].state_dict())
+    ms[1].query_norm.register_forward_hook(lambda *a: None)
+    x = torch.randn(50, 64, device=DEV)
+    real, used = KR.query_norm_backward, []
+    KR.query_norm_backward = lambda *a: (used.append(1), real(*a))[1]
+    try:
+        outs = []
+        for m in ms:
+            stats = m.query_norm.running_mean, m.query_norm.running_var
+            versions = [t._version for t in stats]
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                outs.append(m(x))
+            if m is ms[0]:
+                assert all(t._version > v for t, v in zip(stats, versions))  # what is derived from them is made anew
+            outs[-1].float().square().sum().backward()
+        assert len(used) == 1
+        for name in ("running_mean", "running_var"):
+            assert torch.equal(getattr(ms[0].query_norm, name), getattr(ms[1].query_norm, name))
+        assert int(ms[0].query_norm.num_batches_tracked) == int(ms[1].query_norm.num_batches_tracked) == 1
+        ga, gb = (m.query_norm.weight.grad for m in ms)
+        assert float((ga - gb).norm()) <= 1e-4 * float(gb.norm())
+        assert torch.equal(outs[0], outs[1])                                 # torch's batch norm either way
+        used.clear()
+        ms[0](x).square().sum().backward()                                   # fp32
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            ms[0].query_norm.eval()
+            ms[0](x).float().square().sum().backward()
+            ms[0].query_norm.train()
+            with pytest.raises(ValueError):
+                ms[0](x[:1])                                                 # batch norm of one row
+        assert not used
+    finally:
+        KR.query_norm_backward = real
