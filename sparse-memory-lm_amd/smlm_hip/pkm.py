@@ -13,8 +13,8 @@ Shapes: any n_keys <= 65536 and knn <= min(n_keys, 128) (the reference's torch p
 the reference's power-of-two rule for it.
 
 A forward that autograd records (training) takes the reference's differentiable path with the HIP kernels where the
-reference uses its Triton ones (smlm/pkm.py:186-228): torch query projection and BatchNorm, sub-key scores by
-torch.einsum (its backward is two library GEMMs), the selection and its backward on the kernels (kernels.PKSelect),
+reference uses its Triton ones (smlm/pkm.py:186-228): torch query projection and BatchNorm (its gradient on a kernel in
+bf16), sub-key scores by pk_scores in bf16 and by torch.einsum otherwise (the backward is library GEMMs), the selection and its backward on the kernels (kernels.PKSelect),
 and the values through the row-sparse bag (smlm_hip.sparse_values: fp32 accumulator + touched flags for
 LazyRowAdam) or, with value_grad="dense", F.embedding_bag.
 """
@@ -35,6 +35,51 @@ def _pow2(n):
 
 def _autocast_bf16(x):
     return x.is_cuda and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
+
+
+class _SubkeyScores(torch.autograd.Function):
+    """Both halves' sub-key scores of a bf16 query (N, H, k_dim) in training, recorded as one node: kernels.pk_scores on
+    the keys in bf16, which reads the query and writes (N, H, n_keys) in place (the einsum's batched products copy the
+    query's halves in and the scores out), and a gradient whose products write their part of dq and dkeys in place.  A
+    backward that is itself recorded (create_graph) differentiates the einsum."""
+
+    @staticmethod
+    def forward(ctx, q, keys):
+        k = keys.detach().to(q.dtype).contiguous()
+        ctx.save_for_backward(q, keys, k)
+        return kernels.pk_scores(q, k)
+
+    @staticmethod
+    def backward(ctx, g1, g2):
+        q, keys, k = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            out, grads = zip(*((s, g) for s, g in zip(_score_ops(q, keys.to(q.dtype)), (g1, g2)) if g is not None))
+            wanted = [t for t, n in zip((q, keys), ctx.needs_input_grad) if n]
+            got = iter(torch.autograd.grad(out, wanted, grads, create_graph=True))
+            return tuple(next(got) if n else None for n in ctx.needs_input_grad)
+        need_q, need_k = ctx.needs_input_grad
+        N, H, k_dim = q.shape
+        half = k_dim // 2
+        dq = torch.empty(N, H, 2, half, dtype=q.dtype, device=q.device) if need_q else None
+        dk = torch.empty_like(k) if need_k else None
+        for p, g in enumerate((g1, g2)):
+            if g is None:
+                for t in (dq, dk):
+                    if t is not None:
+                        t.select(2 if t is dq else 1, p).zero_()
+                continue
+            if need_q:
+                torch.bmm(g.transpose(0, 1), k[:, p], out=dq[:, :, p].transpose(0, 1))
+            if need_k:
+                qp = q[..., p * half:(p + 1) * half].transpose(0, 1).contiguous()
+                torch.bmm(g.permute(1, 2, 0), qp, out=dk[:, p])
+        return dq.view(q.shape) if need_q else None, dk.to(keys.dtype) if need_k else None
+
+
+def _score_ops(q, keys):
+    half = q.shape[-1] // 2
+    return (torch.einsum("nhd,hkd->nhk", q[..., :half], keys[:, 0]),
+            torch.einsum("nhd,hkd->nhk", q[..., half:], keys[:, 1]))
 
 
 class _QueryNorm(torch.autograd.Function):
@@ -321,10 +366,13 @@ class ProductKeyMemory(nn.Module):
         q = q.view(N, self.heads, self.k_dim)
         if _autocast_bf16(x):
             q = q.to(torch.bfloat16)
-        half = self.k_dim // 2
-        k1, k2 = self.keys[:, 0], self.keys[:, 1]
-        s1 = torch.einsum("nhd,hkd->nhk", q[..., :half], k1)
-        s2 = torch.einsum("nhd,hkd->nhk", q[..., half:], k2)
+        keys = self.keys
+        if (q.is_cuda and q.dtype == torch.bfloat16 and q.numel() and (self.k_dim // 2) % 8 == 0
+                and (keys.dtype == torch.bfloat16 or (keys.dtype == torch.float32 and _autocast_bf16(x)))
+                and keys.device == q.device and ordinary(q, keys)):
+            s1, s2 = _SubkeyScores.apply(q, keys)
+        else:
+            s1, s2 = _score_ops(q, keys)
         if s1.dtype not in (torch.bfloat16, torch.float32):
             s1, s2 = s1.float(), s2.float()
         scores, indices, weights = kernels.PKSelect.apply(s1, s2, self.knn)

@@ -582,3 +582,42 @@ def test_query_norm_routes():
         assert not used
     finally:
         KR.query_norm_backward = real
+
+
+# ---------------------------------------------------------------------------------------- sub-key scores in training
+@pytest.mark.parametrize("N,H,NK,half,dtype", [(1, 1, 8, 8, torch.float32), (65, 2, 40, 16, torch.float32),
+                                               (200, 4, 512, 256, torch.bfloat16), (1025, 3, 136, 64, torch.float32)])
+def test_subkey_scores_gradient(N, H, NK, half, dtype):
+    """The recorded node against fp64 on the rounded operands: scores and gradients within their bf16 rounding (2^-8) and
+    the fp32 sums' (1e-5 of the largest value); one half's gradient missing; a gradient of the gradient."""
+    note(f"sub-key scores N={N} H={H} NK={NK} half={half} {dtype}")
+    from smlm_hip.pkm import _SubkeyScores
+    g = torch.Generator().manual_seed(N + NK)
+    q = torch.randn(N, H, 2 * half, generator=g).to(torch.bfloat16)
+    keys = (torch.randn(H, 2, NK, half, generator=g) * 0.1).to(torch.bfloat16).to(dtype)
+    gs = [torch.randn(N, H, NK, generator=g).to(torch.bfloat16) for _ in range(2)]
+    ref_in = [t.double().requires_grad_() for t in (q, keys)]
+    ref = [(ref_in[0][..., p * half:(p + 1) * half].transpose(0, 1) @ ref_in[1][:, p].transpose(1, 2)).transpose(0, 1)
+           for p in range(2)]
+    ins = [t.to(DEV).requires_grad_() for t in (q, keys)]
+    got = _SubkeyScores.apply(*ins)
+
+    def close(a, b, extra=0.0):
+        a, b = a.detach().double().cpu(), b.detach()
+        assert bool(((a - b).abs() <= (2 ** -8 + extra) * b.abs() + 1e-5 * b.abs().max()).all())
+
+    for a, b in zip(got, ref):
+        close(a, b)
+    gd = [t.to(DEV) for t in gs]
+    for a, b, t in zip(torch.autograd.grad(got, ins, gd, retain_graph=True),
+                       torch.autograd.grad(ref, ref_in, [t.double() for t in gs], retain_graph=True), ins):
+        assert a.dtype == t.dtype
+        close(a, b)
+    for a, b in zip(torch.autograd.grad(got[1], ins, gd[1], retain_graph=True),
+                    torch.autograd.grad(ref[1], ref_in, gs[1].double(), retain_graph=True)):
+        close(a, b)
+    dq = torch.autograd.grad(got, ins[0], gd, create_graph=True)[0]
+    dd = torch.autograd.grad(dq.float().square().sum(), ins[1])[0].double().cpu()
+    rq = torch.autograd.grad(ref, ref_in[0], [t.double() for t in gs], create_graph=True)[0]
+    rr = torch.autograd.grad(rq.square().sum(), ref_in[1])[0]
+    assert float((dd - rr).norm()) <= 2 ** -6 * float(rr.norm())
