@@ -470,12 +470,13 @@ int smlm_lazy_adam(float *param, void *exp_avg, void *exp_avg_sq, float *exp_avg
 
 /*
  * out[0] = the 2-norm of the rows of acc (rows, D) fp32 with touched[r] != 0 (the accumulator of smlm_bag_backward_*,
- * whose other rows are zero), for the clipping of clip_row_sparse.  Squares and sums in 64 bits, in a fixed order.
+ * whose other rows are zero) and out[1] = min(1, max_norm / (out[0] + 1e-6)), for the clipping of clip_row_sparse.
+ * Squares and sums in 64 bits, in a fixed order.
  * parts: caller-owned scratch of smlm_flagged_norm_parts() doubles, 8-byte aligned.
  */
 int smlm_flagged_norm_parts(void);
-int smlm_flagged_norm(const float *acc, const uint8_t *touched, int64_t rows, int D, double *parts, float *out,
-                      void *stream);
+int smlm_flagged_norm(const float *acc, const uint8_t *touched, int64_t rows, int D, float max_norm, double *parts,
+                      float *out, void *stream);
 
 /*
  * Engram n-gram hash.  Replaces NgramHash.forward (smlm/engram.py:60-73): for every position t of B sequences of

@@ -82,12 +82,16 @@ __global__ void __launch_bounds__(kNormThreads)
 }
 
 // The parts in a fixed order; the sum is rounded to fp32 before the root, so that it overflows where an fp32 sum does.
+// out[1]: the clip factor min(1, max_norm / (norm + 1e-6)) as torch evaluates it (a NaN stays one).
 __global__ void __launch_bounds__(kNormThreads)
-    norm_of_parts_kernel(const double *__restrict__ parts, int n, float *__restrict__ out) {
+    norm_of_parts_kernel(const double *__restrict__ parts, int n, float max_norm, float *__restrict__ out) {
   double sum = 0.0;
   for (int i = threadIdx.x; i < n; i += kNormThreads) sum += parts[i];
   sum = block_sum_f64(sum);
-  if (threadIdx.x == 0) out[0] = sqrtf((float)sum);
+  if (threadIdx.x != 0) return;
+  const float norm = sqrtf((float)sum), factor = 1.0f / (norm + 1e-6f) * max_norm;
+  out[0] = norm;
+  out[1] = factor > 1.0f ? 1.0f : factor;
 }
 
 }  // namespace
@@ -95,8 +99,8 @@ __global__ void __launch_bounds__(kNormThreads)
 
 extern "C" int smlm_flagged_norm_parts(void) { return smlm::kNormParts; }
 
-extern "C" int smlm_flagged_norm(const float *acc, const uint8_t *touched, int64_t rows, int D, double *parts,
-                                 float *out, void *stream) {
+extern "C" int smlm_flagged_norm(const float *acc, const uint8_t *touched, int64_t rows, int D, float max_norm,
+                                 double *parts, float *out, void *stream) {
   using namespace smlm;
   if (!acc || !touched || !parts || !out) return fail(SMLM_EINVAL, "smlm_flagged_norm: null pointer argument");
   if (rows < 0 || D < 1) return fail(SMLM_EINVAL, "smlm_flagged_norm: bad shape rows=%lld D=%d", (long long)rows, D);
@@ -111,6 +115,6 @@ extern "C" int smlm_flagged_norm(const float *acc, const uint8_t *touched, int64
   else
     hipLaunchKernelGGL((flagged_squares_kernel<1>), dim3(blocks), dim3(kNormThreads), 0, s, acc, touched, rows, D, scan,
                        parts);
-  hipLaunchKernelGGL(norm_of_parts_kernel, dim3(1), dim3(kNormThreads), 0, s, parts, blocks, out);
+  hipLaunchKernelGGL(norm_of_parts_kernel, dim3(1), dim3(kNormThreads), 0, s, parts, blocks, max_norm, out);
   return launch_status("smlm_flagged_norm");
 }

@@ -71,7 +71,7 @@ EXPORTS = {
     "smlm_bag_backward_sorted": (_i, [_p, _p, _p, _i64, _i, _p, _i, _i64, _i, _p, _p, _p, _p, _sz, _p]),
     "smlm_lazy_adam": (_i, [_p, _p, _p, _p, _p, _i, _p, _p, _p, _i64, _i, _f, _f, _f, _f, _f, _f, _f, _p]),
     "smlm_flagged_norm_parts": (_i, []),
-    "smlm_flagged_norm": (_i, [_p, _p, _i64, _i, _p, _p, _p]),
+    "smlm_flagged_norm": (_i, [_p, _p, _i64, _i, _f, _p, _p, _p]),
     "smlm_engram_hash": (_i, [_p, _i64, _i64, _i64, _p, _p, _i, _i, _i, _i64, _p, _p]),
     "smlm_engram_mix": (_i, [_p] * 7 + [_i, _p, _p, _i64, _i64, _i, _i, _i, _f, _p, _p]),
     "smlm_engram_mix_parts": (_i64, [_i64, _i64, _i, _i]),

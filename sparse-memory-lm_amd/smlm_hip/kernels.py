@@ -964,19 +964,20 @@ def lazy_adam_step_lowmem(param, exp_avg, exp_avg_sq, acc, touched, grad_scale, 
           exp_avg_sq_scale, "lazy_adam_step_lowmem")
 
 
-def flagged_norm(acc, touched):
-    """2-norm (0-d fp32 tensor) of the rows of acc (rows, D) fp32 flagged in touched (rows,) bool: the norm of a
-    gradient accumulator whose unflagged rows are zero, without reading them (smlm_flagged_norm)."""
+def flagged_norm(acc, touched, max_norm=1.0):
+    """2-norm of the rows of acc (rows, D) fp32 flagged in touched (rows,) bool: the norm of a gradient accumulator whose
+    unflagged rows are zero, without reading them; and the factor min(1, max_norm / (norm + 1e-6)) that clips it
+    (smlm_flagged_norm).  Both 0-d fp32 tensors."""
     _need_cuda("flagged_norm", acc, touched)
     if acc.dtype != torch.float32 or acc.dim() != 2 or not acc.is_contiguous() or touched.dtype != torch.bool \
             or touched.numel() != acc.shape[0] or not touched.is_contiguous():
         raise ValueError("flagged_norm: acc contiguous fp32 (rows, D), touched (rows,) bool")
     parts = torch.empty(_lib.lib().smlm_flagged_norm_parts(), dtype=torch.float64, device=acc.device)
-    out = torch.empty((), dtype=torch.float32, device=acc.device)
-    rc = _lib.lib().smlm_flagged_norm(acc.data_ptr(), touched.data_ptr(), acc.shape[0], acc.shape[1], parts.data_ptr(),
-                                      out.data_ptr(), _stream(acc))
+    out = torch.empty(2, dtype=torch.float32, device=acc.device)
+    rc = _lib.lib().smlm_flagged_norm(acc.data_ptr(), touched.data_ptr(), acc.shape[0], acc.shape[1], float(max_norm),
+                                      parts.data_ptr(), out.data_ptr(), _stream(acc))
     _lib.check(rc, "smlm_flagged_norm")
-    return out
+    return out[0], out[1]
 
 
 def engram_hash(c, mult, orders, rows_per_head):

@@ -314,16 +314,18 @@ def test_flagged_norm(rows, D, read, offset):
     acc = buf[offset:].view(rows, D).normal_(generator=g)
     touched = torch.rand(rows, device=DEV, generator=g) < read
     acc[~touched] = float("nan")
-    got = KR.flagged_norm(acc, touched)
+    got = KR.flagged_norm(acc, touched)[0]
     ref = acc[touched].double().norm().item()
     assert abs(got.item() - ref) <= 2 ** -23 * ref
-    assert all(torch.equal(KR.flagged_norm(acc, touched), got) for _ in range(3))
+    assert all(torch.equal(KR.flagged_norm(acc, touched)[0], got) for _ in range(3))
+    for most in (0.5, 3, 1e9):                          # the clip factor, in torch's arithmetic
+        assert torch.equal(KR.flagged_norm(acc, touched, most)[1], (most / (got + 1e-6)).clamp(max=1.0))
     if touched.any():
         row = int(touched.nonzero()[-1])
         acc[row, -1] = float("inf")
-        assert KR.flagged_norm(acc, touched).item() == float("inf")
+        assert [t.item() for t in KR.flagged_norm(acc, touched)] == [float("inf"), 0.0]
         acc[row, 0] = float("nan")
-        assert D == 1 or torch.isnan(KR.flagged_norm(acc, touched))
+        assert D == 1 or all(torch.isnan(t) for t in KR.flagged_norm(acc, touched))
 
 
 def _adam_case(rows, D, seed):
