@@ -372,6 +372,9 @@ typedef struct smlm_linear_args {
   int64_t hist_len;
   const int64_t *pos;       /* EMBED_ARGMAX with hist: the history slot */
   int64_t *pos_advance;     /* ARGMAX: NULL, or the position to advance by one (M >= 1) */
+  const void *w2;           /* PLAIN with STORE: NULL, or the weight rows [n_split, N), (N - n_split, K) bf16; w then holds the
+                               first n_split */
+  const void *bias2;        /* with w2: their bias (N - n_split,) bf16 or NULL; bias then holds the first n_split */
 } smlm_linear_args;
 
 /* Number of 128-column blocks of the ARGMAX epilogue for N columns (the width partial needs). */

@@ -402,7 +402,8 @@ __device__ __forceinline__ void norm_activations(const smlm_linear_args &a, int6
 
 // PRO / EPI: prologue and epilogue; MAXS: k-steps of 32 per wavefront held in registers (>= its K slice);
 // CPQ: prologue chunks per lane; MTB: token tiles of 16 per workgroup.  ncb column blocks x ntg token groups.
-template <int PRO, int EPI, int MAXS, int CPQ, int MTB>
+// TWO: the columns from n_split on come from a second weight.
+template <int PRO, int EPI, int MAXS, int CPQ, int MTB, bool TWO = false>
 __global__ void __launch_bounds__(kLinThreads) linear_kernel(const smlm_linear_args a, int ncb, int ntg) {
   constexpr bool ARG = EPI == SMLM_LIN_ARGMAX;
   constexpr int KS = ARG ? 1 : kLinWaves;               // wavefronts along the contraction
@@ -430,7 +431,11 @@ __global__ void __launch_bounds__(kLinThreads) linear_kernel(const smlm_linear_a
   const int s_lo = ks * nsteps / KS, ns = (ks + 1) * nsteps / KS - s_lo;
   const int cols = EPI == SMLM_LIN_SWIGLU ? a.N / 2 : a.N;                   // output columns
   const int col0 = ARG ? cb * kArgCols + wave * kArgTiles * 16 : cb * 16;
-  const uint16_t *W = (const uint16_t *)a.w;
+  // n_split % 16 == 0: a 16-column block is on one side.  (A test of w2 in every instance cost a batch-64 decode step
+  // 1.7 us of 176: its weight loads wait for it.)
+  const bool second = TWO && col0 >= a.n_split;
+  const int w_row0 = second ? a.n_split : 0, w_rows = TWO && !second ? a.n_split : a.N - w_row0;
+  const uint16_t *W = (const uint16_t *)(second ? a.w2 : a.w);
 
   // STORE epilogue parameters (bias, affine scale / shift) of wavefront 0's 4 columns, loaded before everything
   // else: read in the epilogue they would add a memory round trip of their own after the products
@@ -440,7 +445,8 @@ __global__ void __launch_bounds__(kLinThreads) linear_kernel(const smlm_linear_a
     if (ks == 0 && c < cols) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        if (a.bias) ep_bias[e] = bf16_bits_to_f32(((const uint16_t *)a.bias)[c + e]);
+        const uint16_t *b = (const uint16_t *)(second ? a.bias2 : a.bias);
+        if (b) ep_bias[e] = bf16_bits_to_f32(b[c - w_row0 + e]);
         if (c < a.n_affine) {
           ep_sc[e] = a.scale[c + e];
           ep_sh[e] = a.shift[c + e];
@@ -467,7 +473,7 @@ __global__ void __launch_bounds__(kLinThreads) linear_kernel(const smlm_linear_a
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     int wrow = EPI == SMLM_LIN_SWIGLU ? (t == 0 ? col0 : cols + col0) + r : col0 + t * 16 + r;
-    wrow = min(wrow, a.N - 1);
+    wrow = min(wrow - w_row0, w_rows - 1);
     const uint16_t *wp = W + (int64_t)wrow * K + g * 8;
 #pragma unroll
     for (int s = 0; s < MAXS; ++s) {
@@ -689,6 +695,13 @@ struct LinGrid {
 
 template <int PRO, int EPI, int MAXS, int MTB>
 void launch_linear_mtb(const smlm_linear_args &a, const LinGrid &lg, hipStream_t stream) {
+  if constexpr (PRO == SMLM_LIN_PLAIN && EPI == SMLM_LIN_STORE) {
+    if (a.w2) {
+      hipLaunchKernelGGL((linear_kernel<PRO, EPI, MAXS, 3, MTB, true>), lg.grid, dim3(kLinThreads), lg.shmem, stream, a,
+                         lg.ncb, lg.ntg);
+      return;
+    }
+  }
   if (PRO == SMLM_LIN_PLAIN || a.K <= 384)
     hipLaunchKernelGGL((linear_kernel<PRO, EPI, MAXS, 3, MTB>), lg.grid, dim3(kLinThreads), lg.shmem, stream, a,
                        lg.ncb, lg.ntg);
@@ -794,6 +807,8 @@ extern "C" int smlm_decode_linear(const smlm_linear_args *a, void *stream) {
     if ((A.n_split > 0 && (!A.out || A.out_stride < A.n_split || A.out_stride % 4 || (uintptr_t)A.out % 8)) ||
         (A.n_split < A.N && (!A.out2 || A.out2_stride < A.N - A.n_split || A.out2_stride % 4 || (uintptr_t)A.out2 % 8)))
       return fail(SMLM_EINVAL, "smlm_decode_linear: out / out2 missing, misaligned or with a short row stride");
+    if (A.w2 ? A.n_split < 16 || A.n_split >= A.N || !aligned16(A.w2) : A.bias2 != nullptr)
+      return fail(SMLM_EINVAL, "smlm_decode_linear: w2 (16-byte aligned) needs 0 < n_split < N; bias2 needs w2");
     if (A.n_affine > 0 && (!A.scale || !A.shift))
       return fail(SMLM_EINVAL, "smlm_decode_linear: n_affine > 0 needs scale and shift");
   } else if (epi == SMLM_LIN_SWIGLU) {
@@ -806,6 +821,8 @@ extern "C" int smlm_decode_linear(const smlm_linear_args *a, void *stream) {
     if (A.pos_advance && A.M == 0)
       return fail(SMLM_EINVAL, "smlm_decode_linear: pos_advance needs M >= 1 (an empty launch runs nothing)");
   }
+  if ((A.w2 || A.bias2) && (epi != SMLM_LIN_STORE || pro != SMLM_LIN_PLAIN))
+    return fail(SMLM_EINVAL, "smlm_decode_linear: w2 and bias2 belong to the PLAIN prologue and STORE epilogue");
   if (A.pos_advance && epi != SMLM_LIN_ARGMAX)
     return fail(SMLM_EINVAL, "smlm_decode_linear: pos_advance belongs to the ARGMAX epilogue");
   if (A.M == 0) return SMLM_OK;

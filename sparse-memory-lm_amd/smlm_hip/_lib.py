@@ -33,6 +33,7 @@ class LinearArgs(ctypes.Structure):
         ("out2_stride", _i64), ("partial", _p), ("partial_stride", _i64), ("delta_parts", _i),
         ("tok_partial", _p), ("tok_partial_stride", _i64), ("tok_blocks", _i), ("tok_out", _p), ("hist", _p),
         ("hist_stride", _i64), ("hist_len", _i64), ("pos", _p), ("pos_advance", _p),
+        ("w2", _p), ("bias2", _p),
     ]
 
 # name -> (restype, argtypes); every function declared in include/smlm_pkm.h

@@ -623,7 +623,7 @@ def _rms_eps(norm):
 
 def decode_linear(weight, x=None, *, delta=None, norm=None, tok=None, emb=None, write_x=False, bias=None,
                   affine=None, n_split=None, swiglu=False, argmax=False, tok_partial=None, tok_out=None, hist=None,
-                  pos=None, partial_out=None, advance_pos=None):
+                  pos=None, partial_out=None, advance_pos=None, weight2=None, bias2=None):
     """Fused small-M linear layer of the decode step (smlm_decode_linear): y = h @ weight.T on the matrix cores.
 
     h is x (M, K) bf16 (unit column stride); with `norm` (an nn.RMSNorm over K with a bf16 weight) it is
@@ -635,7 +635,8 @@ def decode_linear(weight, x=None, *, delta=None, norm=None, tok=None, emb=None, 
     outside the history) when given.  The epilogue is one of
       default   bf16(y + bias) (bias (N,) bf16 or None); `affine` = (scale, shift) fp32 tensors applied as
                 bf16(v * scale + shift) to the first len(scale) columns; with `n_split`, columns [0, n_split) and
-                [n_split, N) are returned as two tensors;
+                [n_split, N) are returned as two tensors; with `weight2` (N2, K) (and `bias2` (N2,) or None) instead of
+                n_split, the two tensors are the projections by weight and by weight2, neither copied;
       swiglu    bf16(bf16(silu(a)) * b) with a | b the two halves of y (weight (2*hidden, K)) -> (M, hidden);
       argmax    no logits: (M, smlm_linear_argmax_blocks(N)) int64 tensor of uint64 partial keys for
                 argmax_finish or the next step's tok_partial (written into `partial_out` when given); with
@@ -647,8 +648,27 @@ def decode_linear(weight, x=None, *, delta=None, norm=None, tok=None, emb=None, 
         raise ValueError("decode_linear: weight must be a contiguous (N, K) bf16 tensor")
     N, K = weight.shape
     args = _lib.LinearArgs()
-    args.N, args.K = N, K
     keep = []
+    if weight2 is not None:
+        _need_cuda("decode_linear", weight2, bias2)
+        if weight2.dtype != torch.bfloat16 or weight2.dim() != 2 or weight2.shape[1] != K or not weight2.is_contiguous() \
+                or n_split is not None or swiglu or argmax or N % 16:
+            raise ValueError("decode_linear: weight2 must be a contiguous (N2, K) bf16 tensor beside a weight of 16 rows or "
+                             "a multiple, without n_split, swiglu or argmax")
+        n_split, n1 = N, N
+        N += weight2.shape[0]
+        args.w2 = weight2.data_ptr()
+        if bias2 is not None:
+            if bias2.dtype != torch.bfloat16 or bias2.numel() != weight2.shape[0]:
+                raise ValueError("decode_linear: bias2 must be (N2,) bf16")
+            bias2 = bias2.contiguous()
+            args.bias2 = bias2.data_ptr()
+        keep += [weight2, bias2]
+    else:
+        n1 = N
+        if bias2 is not None:
+            raise ValueError("decode_linear: bias2 comes with weight2")
+    args.N, args.K = N, K
     if tok is not None or tok_partial is not None:
         if norm is None or emb is None or x is not None or delta is not None or (tok is not None
                                                                                 and tok_partial is not None):
@@ -737,7 +757,7 @@ def decode_linear(weight, x=None, *, delta=None, norm=None, tok=None, emb=None, 
     else:
         args.epilogue = _lib.LIN_STORE
         if bias is not None:
-            if bias.dtype != torch.bfloat16 or bias.numel() != N:
+            if bias.dtype != torch.bfloat16 or bias.numel() != n1:
                 raise ValueError("decode_linear: bias must be (N,) bf16")
             bias = bias.contiguous()
             args.bias = bias.data_ptr()

@@ -393,28 +393,56 @@ class ProductKeyMemory(nn.Module):
             out = self.value_proj(out * F.silu(self.swilu_proj(x)).to(out.dtype))
         return out
 
+    SMALL_BATCH = 64      # rows up to which the projections run on the decode step's kernel
+
+    def _small_batch(self, x):
+        """Whether a no-grad bf16 call's projections run on kernels.decode_linear: few rows, where the library's products
+        and the query's affine are four launches for a few microseconds of work, here two (1 / 16 / 64 tokens, 1024
+        sub-keys, eager: 138 / 124 / 123 -> 79 us; captured and waited for: 63-66 / 60-62 / 70 -> 56-60)."""
+        if not 0 < x.shape[0] <= self.SMALL_BATCH or not self.swilu:
+            return False
+        lins, bn = (self.query_proj, self.swilu_proj, self.value_proj), self.query_norm
+        if not (x.is_cuda and x.dtype == torch.bfloat16 and self.d_in % 32 == 0 and 32 <= self.d_in <= 2048
+                and self.v_dim % 32 == 0 and self.v_dim <= 2048 and self.heads * self.k_dim % 16 == 0 and self.d_out % 16 == 0 and (bn is None or not bn.training)
+                and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)):
+            return False
+        for lin in lins:
+            w, b = lin.weight, lin.bias
+            if not (type(lin) is nn.Linear and w.dtype == torch.bfloat16 and w.device == x.device and w.is_contiguous()
+                    and w.data_ptr() % 16 == 0 and (b is None or (b.dtype == torch.bfloat16 and b.device == x.device))):
+                return False
+        return unhooked(*lins) and ordinary(x) and not records(x, *(lin.weight for lin in lins))
+
     def _forward(self, x):
         if torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters())):
             return self._train_forward(x)
         N = x.shape[0]
         bf16 = _autocast_bf16(x) or x.dtype == torch.bfloat16
         sdt = torch.bfloat16 if (bf16 or self.keys.dtype == torch.bfloat16) else torch.float32
-        q = self._query(x).to(sdt).view(N, self.heads, self.k_dim)
+        pre, value_proj = None, kernels.linear
+        if self._small_batch(x):
+            # the query with its BatchNorm and the swilu input in one launch, and value_proj, on the decode step's kernel
+            affine = self._bn_affine() if self.query_norm is not None else None
+            q, pre = kernels.decode_linear(self.query_proj.weight, x, bias=self.query_proj.bias, affine=affine,
+                                           weight2=self.swilu_proj.weight, bias2=self.swilu_proj.bias)
+            q = q.view(N, self.heads, self.k_dim)
+            value_proj = lambda mod, out: kernels.decode_linear(mod.weight, out, bias=mod.bias)  # noqa: E731
+        else:
+            q = self._query(x).to(sdt).view(N, self.heads, self.k_dim)
         s1, s2 = kernels.pk_scores(q, self._keys_as(sdt))
         tables = inference_tables(self.values) if self.swilu and bf16 else None
         if (tables is not None and self.log_score_scale is None
                 and kernels.select_bag_supported(self.heads, tables[0], tables[1])):
             # selection, value bag and swilu epilogue in one launch (the same results as pk_select then bag_infer;
             # different workgroups overlap the selection's vector work with the gather's memory traffic)
-            pre = kernels.linear(self.swilu_proj, x).to(torch.bfloat16)
+            pre = kernels.linear(self.swilu_proj, x).to(torch.bfloat16) if pre is None else pre
             res = kernels.pk_select_bag(s1, s2, self.knn, tables[0], tables[1], pre=pre, out_bf16=True,
                                         record=self.record)
             out = res[0] if self.record else res
             if self.record:
                 self.last_scores, self.last_indices, self.last_weights = res[1], res[2], res[3]
                 self.last_lookup = {"x": x, "q": q, "s1": s1, "s2": s2}
-            return kernels.linear(self.value_proj,
-                                  out.to(self.value_proj.weight.dtype) if not _autocast_bf16(x) else out)
+            return value_proj(self.value_proj, out.to(self.value_proj.weight.dtype) if not _autocast_bf16(x) else out)
         scores, indices, weights = kernels.pk_select(s1, s2, self.knn)
         if self.log_score_scale is not None:
             # a positive per-head scale keeps the selection; only the softmax sharpness changes
@@ -426,14 +454,13 @@ class ProductKeyMemory(nn.Module):
         idx, w = indices.view(N, -1), weights.view(N, -1)
         if self.swilu and bf16:
             # fused inference bag: value rows (bf16 / fp32 / int8 / q4 table) * bf16(silu(pre)), bf16 out
-            pre = kernels.linear(self.swilu_proj, x).to(torch.bfloat16)
+            pre = kernels.linear(self.swilu_proj, x).to(torch.bfloat16) if pre is None else pre
             tables = inference_tables(self.values)
             if tables is None:                  # a table tier that stages every call (smlm_hip.offload)
                 out = self.values.infer_table.bag(idx, w, pre)
             else:
                 out = kernels.bag_infer(idx, w, tables[0], tables[1], pre=pre, out_bf16=True)
-            return kernels.linear(self.value_proj,
-                                  out.to(self.value_proj.weight.dtype) if not _autocast_bf16(x) else out)
+            return value_proj(self.value_proj, out.to(self.value_proj.weight.dtype) if not _autocast_bf16(x) else out)
         out = self.read_values(idx, w)
         if self.swilu:
             out = self.value_proj(out * F.silu(self.swilu_proj(x)).to(out.dtype))

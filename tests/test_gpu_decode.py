@@ -511,3 +511,63 @@ def test_fused_step_with_memory_layer_matches_torch_path(monkeypatch, proj_max, 
                             selections={mem_layer: (idx.cpu(), w.cpu())})[:, -1]
         err = float((got - ref).abs().max() / ref.abs().max())
         assert err < 1e-2, err
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 33, 64])
+@pytest.mark.parametrize("K_in,N1,N2,biased", [(384, 2048, 384, True), (32, 16, 16, True), (96, 48, 208, False)])
+def test_decode_linear_of_two_weights(M, K_in, N1, N2, biased):
+    """Columns from two weights that lie apart: the same bits as a launch for each, with their biases and the affine on
+    the first."""
+    g = torch.Generator().manual_seed(M + K_in)
+    x = torch.randn(M, K_in, generator=g).to(DEV, torch.bfloat16)
+    ws = [(torch.randn(n, K_in, generator=g) * K_in ** -0.5).to(DEV, torch.bfloat16) for n in (N1, N2)]
+    bs = [torch.randn(n, generator=g).to(DEV, torch.bfloat16) if biased else None for n in (N1, N2)]
+    affine = tuple(torch.rand(N1, generator=g).to(DEV) + 0.5 for _ in range(2))
+    got = K.decode_linear(ws[0], x, bias=bs[0], affine=affine, weight2=ws[1], bias2=bs[1])
+    assert torch.equal(got[0], K.decode_linear(ws[0], x, bias=bs[0], affine=affine))
+    assert torch.equal(got[1], K.decode_linear(ws[1], x, bias=bs[1]))
+    for bad in (dict(weight2=ws[1], n_split=16), dict(weight2=ws[1], argmax=True), dict(bias2=bs[1] if biased else ws[1][0])):
+        with pytest.raises(ValueError):
+            K.decode_linear(ws[0], x, **bad)
+
+
+@torch.no_grad()
+def test_memory_layer_small_batches_take_the_decode_kernel():
+    """Up to 64 rows in bf16 the layer's projections run on the decode step's kernel, with the query's affine and
+    value_proj: the same numbers as the other route within bf16, with and without autocast and a score scale; hooks,
+    fp32 and more rows keep the modules."""
+    from smlm_hip.pkm import ProductKeyMemory
+    torch.manual_seed(0)
+    real, used = K.decode_linear, []
+    K.decode_linear = lambda *a, **kw: (used.append(1), real(*a, **kw))[1]
+    try:
+        for kw in ({}, {"score_scale": "learned"}, {"query_norm": "none"}):
+            m = ProductKeyMemory(64, 64, n_keys=64, heads=2, knn=8, k_dim=64, **kw).to(DEV).eval()
+            if m.query_norm is not None:
+                m.query_norm.running_var.uniform_(0.5, 1.5)
+                m.query_norm.running_mean.normal_(0, 0.1)
+            m = m.to(torch.bfloat16)
+            x = torch.randn(64, 64, device=DEV, dtype=torch.bfloat16)
+            for autocast in (False, True):
+                with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+                    used.clear()
+                    small = torch.cat([m(x[:1]), m(x[1:])])
+                    assert len(used) == 4
+                    m.SMALL_BATCH = 0
+                    used.clear()
+                    other = m(x)
+                    assert not used
+                    del m.SMALL_BATCH
+                    assert small.dtype == other.dtype
+                    # a rounded query or score may change a few of the 1,024 selections
+                    assert float((small - other).float().norm()) <= 0.1 * float(other.float().norm())
+                    assert float(((small - other).float().abs().amax(-1) <= 2 ** -5 * other.float().abs().max()).float().mean()) >= 0.9
+        used.clear()
+        m(torch.randn(65, 64, device=DEV, dtype=torch.bfloat16))
+        hook = m.value_proj.register_forward_hook(lambda *a: None)
+        m(x)
+        hook.remove()
+        m.float()(x.float())
+        assert not used
+    finally:
+        K.decode_linear = real
