@@ -268,8 +268,8 @@ class SwiGLU(nn.Module):
     fused_min_rows = 128   # prompt passes: rows from which the projection and activation are one launch
 
     def forward(self, x):
-        """w2(silu(a) * b) with a | b = w13(x).  On bf16 GPU tensors the activation is one kernel
-        (smlm_hip.kernels.swiglu) with the same roundings; without autograd, from fused_min_rows rows on, the w13
+        """w2(silu(a) * b) with a | b = w13(x).  On bf16 GPU tensors without autograd the activation is one
+        kernel (smlm_hip.kernels.swiglu) with the same roundings; from fused_min_rows rows on, the w13
         projection and the activation are one launch (kernels.linear_swiglu: the same roundings, and the
         projection's products on the matrix cores in fp32), and w2 runs through kernels.linear."""
         w = self.w13.weight
@@ -279,7 +279,7 @@ class SwiGLU(nn.Module):
                 and not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16)):
             return kernels.linear(self.w2, kernels.linear_swiglu(x, w))
         h = self.w13(x)
-        if h.is_cuda and h.dtype == torch.bfloat16 and h.shape[-1] % 16 == 0:
+        if h.is_cuda and h.dtype == torch.bfloat16 and h.shape[-1] % 16 == 0 and not records(h):
             act = kernels.swiglu(h)
         else:
             a, b = h.chunk(2, dim=-1)
@@ -420,7 +420,7 @@ class Transformer(nn.Module):
         x = self.tok_emb(idx)
         rows = self._ngram_rows(idx, kv_caches) if self.ngram is not None else None
         if (x.is_cuda and x.dtype == torch.bfloat16 and not torch.is_autocast_enabled("cuda")
-                and self.ngram is None):
+                and self.ngram is None and not records(x, *self.parameters())):
             logits = self.lm_head(self._blocks_fused_norms(x, kv_caches, pos0))
         else:
             for i, blk in enumerate(self.layers):

@@ -335,3 +335,24 @@ def test_generate_with_reference_torch_shapes():
     rs, ri, rw = O.pk_select(bits_of(r["s1"]), bits_of(r["s2"]), 5)
     assert np.array_equal(r["indices"].cpu().numpy(), ri) and np.array_equal(bits_of(r["scores"]), rs)
     np.testing.assert_allclose(r["weights"].cpu().numpy(), rw, rtol=0, atol=1e-6)
+
+
+@pytest.mark.parametrize("weights,autocast", [(torch.float32, True), (torch.bfloat16, False), (torch.float32, False)])
+def test_every_dense_parameter_of_the_lm_gets_its_gradient(weights, autocast):
+    """A recorded forward with targets reaches every parameter, in fp32, under bf16 autocast and on bf16 weights (the
+    forward-only kernels of prompt passes stay out of it): gradients near those of the fp32 model on the CPU."""
+    print(f"lm gradients {weights} autocast={autocast}", flush=True)
+    torch.manual_seed(0)
+    ref = Transformer(ModelConfig(vocab_size=320, d_model=64, n_layers=2, n_heads=2, ffn_hidden=64, max_seq_len=48))
+    m = Transformer(ref.cfg)
+    m.load_state_dict(ref.state_dict())
+    m = m.to("cuda", weights)
+    x = torch.randint(0, 320, (2, 48))
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+        loss = m(x.cuda(), x.roll(-1, 1).cuda())[1]
+    loss.backward()
+    ref(x, x.roll(-1, 1))[1].backward()
+    for (name, p), q in zip(m.named_parameters(), ref.parameters()):
+        assert p.grad is not None, name
+        err = float((p.grad.float().cpu() - q.grad).norm() / q.grad.norm())
+        assert err <= (1e-3 if weights == torch.float32 and not autocast else 0.1), (name, err)
