@@ -401,9 +401,14 @@ class ProductKeyMemory(nn.Module):
         sub-keys, eager: 138 / 124 / 123 -> 79 us; captured and waited for: 63-66 / 60-62 / 70 -> 56-60)."""
         if not 0 < x.shape[0] <= self.SMALL_BATCH or not self.swilu:
             return False
+        # the kernel reads rows of its own, 16 bytes at a time: a repeated row (expand) or one off its alignment (a slice)
+        # stays with the modules
+        if x.stride(1) != 1 or x.stride(0) < self.d_in or x.stride(0) % 8 or x.data_ptr() % 16:
+            return False
         lins, bn = (self.query_proj, self.swilu_proj, self.value_proj), self.query_norm
         if not (x.is_cuda and x.dtype == torch.bfloat16 and self.d_in % 32 == 0 and 32 <= self.d_in <= 2048
-                and self.v_dim % 32 == 0 and self.v_dim <= 2048 and self.heads * self.k_dim % 16 == 0 and self.d_out % 16 == 0 and (bn is None or not bn.training)
+                and self.v_dim % 32 == 0 and self.v_dim <= 2048 and self.heads * self.k_dim % 16 == 0
+                and self.d_out % 16 == 0 and (bn is None or not bn.training)
                 and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)):
             return False
         for lin in lins:

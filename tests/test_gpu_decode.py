@@ -571,3 +571,19 @@ def test_memory_layer_small_batches_take_the_decode_kernel():
         assert not used
     finally:
         K.decode_linear = real
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("layout", ["repeated row", "one repeated row", "odd offset", "odd stride", "column stride"])
+def test_memory_layer_small_batches_of_any_layout(layout):
+    """A few rows that the decode step's kernel does not read as they lie (a stride below the width, off 16 bytes) give
+    the result of their contiguous copy, up to bf16 (two products, and a selection moved by a rounded score)."""
+    from smlm_hip.pkm import ProductKeyMemory
+    torch.manual_seed(0)
+    m = ProductKeyMemory(64, 64, n_keys=64, heads=2, knn=8, k_dim=64).to(DEV).eval().to(torch.bfloat16)
+    flat = torch.randn(9 * 72, device=DEV, dtype=torch.bfloat16)
+    x = {"repeated row": flat[:64].expand(5, 64), "one repeated row": flat[:64].expand(1, 64),
+         "odd offset": flat[1:1 + 5 * 64].view(5, 64), "odd stride": flat[:5 * 67].view(5, 67)[:, :64],
+         "column stride": flat[:5 * 128].view(5, 64, 2)[..., 0]}[layout]
+    got, ref = m(x).float(), m(x.contiguous().clone()).float()
+    assert got.shape == ref.shape and float((got - ref).norm()) <= 0.1 * float(ref.norm())
