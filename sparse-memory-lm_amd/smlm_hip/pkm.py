@@ -45,9 +45,9 @@ class _SubkeyScores(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, keys):
-        k = keys.detach().to(q.dtype).contiguous()
+        k = kernels._aligned(keys.detach().to(q.dtype))    # bf16 keys may be a view into a flat buffer
         ctx.save_for_backward(q, keys, k)
-        return kernels.pk_scores(q, k)
+        return kernels.pk_scores(kernels._aligned(q), k)
 
     @staticmethod
     def backward(ctx, g1, g2):

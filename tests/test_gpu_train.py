@@ -623,3 +623,21 @@ def test_subkey_scores_gradient(N, H, NK, half, dtype):
     rq = torch.autograd.grad(ref, ref_in[0], [t.double() for t in gs], create_graph=True)[0]
     rr = torch.autograd.grad(rq.square().sum(), ref_in[1])[0]
     assert float((dd - rr).norm()) <= 2 ** -6 * float(rr.norm())
+
+
+def test_subkey_scores_of_keys_off_16_bytes():
+    """bf16 keys and queries that are views into flat buffers at an odd offset: the result and gradients of their copies,
+    bit for bit (the kernel reads 16-byte aligned copies)."""
+    note("sub-key scores of keys off 16 bytes")
+    from smlm_hip.pkm import _SubkeyScores
+    g = torch.Generator().manual_seed(3)
+    flat = torch.randn(2 * 2 * 40 * 16 + 33 * 2 * 32 + 1, generator=g).to(DEV, torch.bfloat16)
+    keys, q = flat[1:1 + 2 * 2 * 40 * 16].view(2, 2, 40, 16), flat[1 + 2 * 2 * 40 * 16:].view(33, 2, 32)
+    assert keys.data_ptr() % 16 and q.data_ptr() % 16
+    both = []
+    for ins in ((q.detach(), keys.detach()), (q.clone(), keys.clone())):
+        ins = [t.requires_grad_() for t in ins]
+        out = _SubkeyScores.apply(*ins)
+        both.append((*out, *torch.autograd.grad(out, ins, [torch.ones_like(t) for t in out])))
+    for a, b in zip(*both):
+        assert torch.equal(a, b)
