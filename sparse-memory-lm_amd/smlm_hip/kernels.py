@@ -428,7 +428,7 @@ def attention_train(qkv, rope_cos, rope_sin, pos0, H):
     RoPE at positions pos0 .. (rope_qkv) and prefill_attention, returning (y (B, T, H*hd) bf16, q and k after RoPE
     (B, H, T, hd), lse (B*H, T rounded up to 64) fp32)."""
     _need_cuda("attention_train", qkv)
-    qkv = qkv.contiguous()
+    qkv, rope_cos, rope_sin = _aligned(qkv), _aligned(rope_cos), _aligned(rope_sin)
     B, T, C3 = qkv.shape
     hd = C3 // (3 * H)
     if C3 != 3 * H * hd or hd not in (32, 64, 128):
@@ -457,7 +457,7 @@ def attention_backward(dy, qkv, y, q, k, lse, rope_cos, rope_sin, pos0):
     if rope_cos.dtype not in _DT or rope_sin.dtype != rope_cos.dtype or rope_cos.shape != rope_sin.shape \
             or rope_cos.dim() != 2 or rope_cos.shape[1] != hd // 2:
         raise ValueError("attention_backward: rope tables must be (max_seq_len, head_dim/2) fp32 or bf16")
-    qkv, dy, rope_cos, rope_sin = qkv.contiguous(), _aligned(dy), rope_cos.contiguous(), rope_sin.contiguous()
+    qkv, dy, rope_cos, rope_sin = _aligned(qkv), _aligned(dy), rope_cos.contiguous(), rope_sin.contiguous()
     v, dqkv, delta = _v_of(qkv, H), torch.empty_like(qkv), torch.empty_like(lse)
     vs = (ctypes.c_int64 * 3)(v.stride(0), v.stride(2), v.stride(1))
     ys = (ctypes.c_int64 * 3)(T * H * hd, hd, H * hd)

@@ -478,3 +478,23 @@ def test_attention_training_routes():
         assert run()[1] == 0
     assert run(kv_cache={})[1] == 0
     assert a(x).dtype == torch.float32 and not used[1:]
+
+
+def test_attention_training_of_a_projection_off_16_bytes():
+    """A qkv projection that is a view into a flat buffer at an odd offset (a hook's result, say) has the result and the
+    gradient of its copy, bit for bit."""
+    print("attention training off 16 bytes", flush=True)
+    from smlm_hip.model import RotaryEmbedding, _AttentionTrain
+    g = torch.Generator().manual_seed(4)
+    rope = RotaryEmbedding(32, 70, 10000.0).to(DEV)
+    flat = torch.randn(2 * 70 * 192 + 1, generator=g).to(DEV, torch.bfloat16)
+    qkv = flat[1:].view(2, 70, 192)
+    dy = torch.randn(2, 70, 64, generator=g).to(DEV, torch.bfloat16)
+    assert qkv.data_ptr() % 16
+    both = []
+    for t in (qkv.detach(), qkv.clone()):
+        t.requires_grad_()
+        y = _AttentionTrain.apply(t, rope, 0, 2)
+        both.append((y, torch.autograd.grad(y, t, dy)[0]))
+    for a, b in zip(*both):
+        assert torch.equal(a, b)
