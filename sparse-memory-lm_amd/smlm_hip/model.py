@@ -420,7 +420,7 @@ class Transformer(nn.Module):
         x = self.tok_emb(idx)
         rows = self._ngram_rows(idx, kv_caches) if self.ngram is not None else None
         if (x.is_cuda and x.dtype == torch.bfloat16 and not torch.is_autocast_enabled("cuda")
-                and self.ngram is None and not records(x, *self.parameters())):
+                and self.ngram is None and not (torch.is_grad_enabled() and records(x, *self.parameters()))):
             logits = self.lm_head(self._blocks_fused_norms(x, kv_caches, pos0))
         else:
             for i, blk in enumerate(self.layers):
