@@ -416,6 +416,14 @@ int smlm_query_norm_backward(const void *g, const void *x, const float *weight, 
                              void *stream);
 
 /*
+ * Gradient of smlm_pkm_score's keys in training (smlm/pkm.py:117-123): dk[h, p, k, :] = sum_n g_p[n, h, k] q[n, h, p half
+ * + :] from g1, g2 (N, H, NK) and q (N, H, 2 half) bf16 contiguous into dk (H, 2, NK, half) fp32 or bf16 (fp32 sums); a null
+ * g1 or g2 gives zeros.  NK and half multiples of 8; every tensor 16-byte aligned and its rows within 2 GB.
+ */
+int smlm_score_keys_grad(const void *g1, const void *g2, const void *q, int64_t N, int H, int NK, int half, void *dk,
+                         int dk_dtype, void *stream);
+
+/*
  * Row-sparse value-bag backward (smlm/kernels.py:1-104, smlm/sparse_values.py:94-113):
  *   acc[idx[n,k], :] += w[n,k] * grad_out[n, :]   (fp32 atomic adds: the order of additions is not fixed)
  *   touched[idx[n,k]] = 1

@@ -65,6 +65,7 @@ EXPORTS = {
     "smlm_decode_linear": (_i, [ctypes.POINTER(LinearArgs), _p]),
     "smlm_argmax_finish": (_i, [_p, _i64, _i, _i64, _p, _p, _p, _i64, _i64, _i, _p]),
     "smlm_pkm_select_backward": (_i, [_p, _p, _p, _p, _i, _i64, _i, _i, _i, _p, _p, _p]),
+    "smlm_score_keys_grad": (_i, [_p, _p, _p, _i64, _i, _i, _i, _p, _i, _p]),
     "smlm_query_norm_parts": (_i64, [_i64, _i]),
     "smlm_query_norm_backward": (_i, [_p] * 5 + [_i64, _i] + [_p] * 6),
     "smlm_bag_backward_rows": (_i, [_p, _p, _p, _i64, _i, _p, _i, _i64, _i, _p, _p, _p, _p]),

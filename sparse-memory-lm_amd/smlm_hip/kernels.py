@@ -857,6 +857,30 @@ class PKSelect(torch.autograd.Function):
         return ds1, ds2, None
 
 
+def score_keys_grad_supported(N, H, NK, half):
+    """Whether score_keys_grad takes these shapes: whole 16-byte chunks, byte offsets of 32 bits."""
+    return N > 0 and NK % 8 == 0 and half % 8 == 0 and (N + 320) * H * max(NK, 2 * half) * 2 + 512 < 2 ** 31
+
+
+def score_keys_grad(g1, g2, q, keys_shape, dtype):
+    """Gradient (H, 2, NK, half) of pk_scores' keys in `dtype` (fp32 or bf16, from fp32 sums) from the score gradients g1, g2
+    (N, H, NK) bf16 (None: zeros in its half) and q (N, H, 2 * half) bf16.  The same result on every call."""
+    _need_cuda("score_keys_grad", g1, g2, q)
+    H, two, NK, half = keys_shape
+    N = q.shape[0]
+    if q.dtype != torch.bfloat16 or tuple(q.shape) != (N, H, 2 * half) or two != 2 or dtype not in _DT:
+        raise ValueError(f"score_keys_grad: q must be (N, {H}, {2 * half}) bf16 and the result fp32 or bf16")
+    for g in (g1, g2):
+        if g is not None and (g.dtype != torch.bfloat16 or tuple(g.shape) != (N, H, NK)):
+            raise ValueError(f"score_keys_grad: gradients must be ({N}, {H}, {NK}) bf16")
+    g1, g2, q = (t if t is None else _aligned(t) for t in (g1, g2, q))
+    dk = torch.empty(H, 2, NK, half, dtype=dtype, device=q.device)
+    rc = _lib.lib().smlm_score_keys_grad(None if g1 is None else g1.data_ptr(), None if g2 is None else g2.data_ptr(),
+                                         q.data_ptr(), N, H, NK, half, dk.data_ptr(), _DT[dtype], _stream(q))
+    _lib.check(rc, "smlm_score_keys_grad")
+    return dk
+
+
 def query_norm_backward(g, x, weight, mean, invstd):
     """Gradient of the memory query's batch norm in training (smlm/pkm.py:188-191) from g and x (N >= 2, C) bf16, weight
     and the forward's mean and 1 / sqrt(var + eps) (C,) fp32: (dx (N, C) bf16, dweight, dbias (C,) fp32).  C a multiple

@@ -40,8 +40,9 @@ def _autocast_bf16(x):
 class _SubkeyScores(torch.autograd.Function):
     """Both halves' sub-key scores of a bf16 query (N, H, k_dim) in training, recorded as one node: kernels.pk_scores on
     the keys in bf16, which reads the query and writes (N, H, n_keys) in place (the einsum's batched products copy the
-    query's halves in and the scores out), and a gradient whose products write their part of dq and dkeys in place.  A
-    backward that is itself recorded (create_graph) differentiates the einsum."""
+    query's halves in and the scores out), and a gradient whose products write their part of dq in place and whose dkeys
+    are one launch (kernels.score_keys_grad; n_keys that are no multiple of 8: products too).  A backward that is itself
+    recorded (create_graph) differentiates the einsum."""
 
     @staticmethod
     def forward(ctx, q, keys):
@@ -61,7 +62,11 @@ class _SubkeyScores(torch.autograd.Function):
         N, H, k_dim = q.shape
         half = k_dim // 2
         dq = torch.empty(N, H, 2, half, dtype=q.dtype, device=q.device) if need_q else None
-        dk = torch.empty_like(k) if need_k else None
+        dk, whole = None, None
+        if need_k and kernels.score_keys_grad_supported(N, H, k.shape[2], half):
+            whole, need_k = kernels.score_keys_grad(g1, g2, q, k.shape, keys.dtype), False
+        elif need_k:
+            dk = torch.empty_like(k)
         for p, g in enumerate((g1, g2)):
             if g is None:
                 for t in (dq, dk):
@@ -73,7 +78,7 @@ class _SubkeyScores(torch.autograd.Function):
             if need_k:
                 qp = q[..., p * half:(p + 1) * half].transpose(0, 1).contiguous()
                 torch.bmm(g.permute(1, 2, 0), qp, out=dk[:, p])
-        return dq.view(q.shape) if need_q else None, dk.to(keys.dtype) if need_k else None
+        return dq.view(q.shape) if need_q else None, dk.to(keys.dtype) if need_k else whole
 
 
 def _score_ops(q, keys):

@@ -588,7 +588,8 @@ def test_query_norm_routes():
 
 # ---------------------------------------------------------------------------------------- sub-key scores in training
 @pytest.mark.parametrize("N,H,NK,half,dtype", [(1, 1, 8, 8, torch.float32), (65, 2, 40, 16, torch.float32),
-                                               (200, 4, 512, 256, torch.bfloat16), (1025, 3, 136, 64, torch.float32)])
+                                               (200, 4, 512, 256, torch.bfloat16), (1025, 3, 136, 64, torch.float32), (33, 2, 12, 16, torch.float32),
+                                               (300, 1, 72, 136, torch.bfloat16)])
 def test_subkey_scores_gradient(N, H, NK, half, dtype):
     """The recorded node against fp64 on the rounded operands: scores and gradients within their bf16 rounding (2^-8) and
     the fp32 sums' (1e-5 of the largest value); one half's gradient missing; a gradient of the gradient."""
