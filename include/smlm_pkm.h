@@ -372,15 +372,19 @@ typedef struct smlm_linear_args {
   int64_t hist_len;
   const int64_t *pos;       /* EMBED_ARGMAX with hist: the history slot */
   int64_t *pos_advance;     /* ARGMAX: NULL, or the position to advance by one (M >= 1) */
-  const void *w2;           /* PLAIN with STORE: NULL, or the weight rows [n_split, N), (N - n_split, K) bf16; w then holds the
-                               first n_split */
-  const void *bias2;        /* with w2: their bias (N - n_split,) bf16 or NULL; bias then holds the first n_split */
 } smlm_linear_args;
 
 /* Number of 128-column blocks of the ARGMAX epilogue for N columns (the width partial needs). */
 int smlm_linear_argmax_blocks(int N);
 
 int smlm_decode_linear(const smlm_linear_args *args, void *stream);
+
+/*
+ * smlm_decode_linear with the PLAIN prologue and STORE epilogue over two weights: the columns [0, n_split) by args->w
+ * (n_split, K) and args->bias, [n_split, N) by w2 (N - n_split, K) bf16, 16-byte aligned, and bias2 (N - n_split,) bf16 or
+ * NULL; 0 < n_split < N.
+ */
+int smlm_decode_linear_pair(const smlm_linear_args *args, const void *w2, const void *bias2, void *stream);
 
 /*
  * End of a greedy decode step (smlm/train.py:297-301: nxt = logits.argmax(-1), appended to the sequence), in one

@@ -36,6 +36,8 @@
 //
 // MFMA operand mapping (16x16x32, r = lane % 16, g = lane / 16): A = 16 weight rows x 32 k (lane: row r, k group g),
 // B = 32 k x 16 tokens (lane: token r, k group g), D: lane holds columns 4g..4g+3 of token r.
+#include <type_traits>
+
 #include "pkm_common.h"
 
 namespace smlm {
@@ -403,8 +405,13 @@ __device__ __forceinline__ void norm_activations(const smlm_linear_args &a, int6
 // PRO / EPI: prologue and epilogue; MAXS: k-steps of 32 per wavefront held in registers (>= its K slice);
 // CPQ: prologue chunks per lane; MTB: token tiles of 16 per workgroup.  ncb column blocks x ntg token groups.
 // TWO: the columns from n_split on come from a second weight.
+struct LinNone {};
+struct LinSecond {
+  const void *w, *bias;
+};
 template <int PRO, int EPI, int MAXS, int CPQ, int MTB, bool TWO = false>
-__global__ void __launch_bounds__(kLinThreads) linear_kernel(const smlm_linear_args a, int ncb, int ntg) {
+__global__ void __launch_bounds__(kLinThreads) linear_kernel(
+    const smlm_linear_args a, int ncb, int ntg, std::conditional_t<TWO, LinSecond, LinNone> other) {
   constexpr bool ARG = EPI == SMLM_LIN_ARGMAX;
   constexpr int KS = ARG ? 1 : kLinWaves;               // wavefronts along the contraction
   constexpr int NT = EPI == SMLM_LIN_STORE ? 1 : 2;     // weight tiles per wavefront
@@ -435,7 +442,11 @@ __global__ void __launch_bounds__(kLinThreads) linear_kernel(const smlm_linear_a
   // 1.7 us of 176: its weight loads wait for it.)
   const bool second = TWO && col0 >= a.n_split;
   const int w_row0 = second ? a.n_split : 0, w_rows = TWO && !second ? a.n_split : a.N - w_row0;
-  const uint16_t *W = (const uint16_t *)(second ? a.w2 : a.w);
+  const uint16_t *W = (const uint16_t *)a.w;
+  const uint16_t *bias = (const uint16_t *)a.bias;
+  if constexpr (TWO) {
+    if (second) W = (const uint16_t *)other.w, bias = (const uint16_t *)other.bias;
+  }
 
   // STORE epilogue parameters (bias, affine scale / shift) of wavefront 0's 4 columns, loaded before everything
   // else: read in the epilogue they would add a memory round trip of their own after the products
@@ -445,8 +456,7 @@ __global__ void __launch_bounds__(kLinThreads) linear_kernel(const smlm_linear_a
     if (ks == 0 && c < cols) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const uint16_t *b = (const uint16_t *)(second ? a.bias2 : a.bias);
-        if (b) ep_bias[e] = bf16_bits_to_f32(b[c - w_row0 + e]);
+        if (bias) ep_bias[e] = bf16_bits_to_f32(bias[c - w_row0 + e]);
         if (c < a.n_affine) {
           ep_sc[e] = a.scale[c + e];
           ep_sh[e] = a.shift[c + e];
@@ -688,6 +698,7 @@ __global__ void __launch_bounds__(kFinishThreads)
 
 // Launch geometry: ncb column blocks x ntg token groups of mtb tiles.
 struct LinGrid {
+  LinSecond second;
   int ncb, ntg, mtb;
   dim3 grid;
   size_t shmem;
@@ -696,18 +707,18 @@ struct LinGrid {
 template <int PRO, int EPI, int MAXS, int MTB>
 void launch_linear_mtb(const smlm_linear_args &a, const LinGrid &lg, hipStream_t stream) {
   if constexpr (PRO == SMLM_LIN_PLAIN && EPI == SMLM_LIN_STORE) {
-    if (a.w2) {
+    if (lg.second.w) {
       hipLaunchKernelGGL((linear_kernel<PRO, EPI, MAXS, 3, MTB, true>), lg.grid, dim3(kLinThreads), lg.shmem, stream, a,
-                         lg.ncb, lg.ntg);
+                         lg.ncb, lg.ntg, lg.second);
       return;
     }
   }
   if (PRO == SMLM_LIN_PLAIN || a.K <= 384)
     hipLaunchKernelGGL((linear_kernel<PRO, EPI, MAXS, 3, MTB>), lg.grid, dim3(kLinThreads), lg.shmem, stream, a,
-                       lg.ncb, lg.ntg);
+                       lg.ncb, lg.ntg, LinNone{});
   else
     hipLaunchKernelGGL((linear_kernel<PRO, EPI, MAXS, 4, MTB>), lg.grid, dim3(kLinThreads), lg.shmem, stream, a,
-                       lg.ncb, lg.ntg);
+                       lg.ncb, lg.ntg, LinNone{});
 }
 
 template <int PRO, int EPI, int MAXS>
@@ -743,13 +754,7 @@ void launch_linear_pro(const smlm_linear_args &a, const LinGrid &grid, hipStream
 
 bool aligned16(const void *p) { return ((uintptr_t)p % 16) == 0; }
 
-}  // namespace
-}  // namespace smlm
-
-extern "C" int smlm_linear_argmax_blocks(int N) { return N <= 0 ? 0 : (N + smlm::kArgCols - 1) / smlm::kArgCols; }
-
-extern "C" int smlm_decode_linear(const smlm_linear_args *a, void *stream) {
-  using namespace smlm;
+int decode_linear(const smlm_linear_args *a, const LinSecond second, void *stream) {
   if (!a) return fail(SMLM_EINVAL, "smlm_decode_linear: null argument block");
   const smlm_linear_args &A = *a;
   const int pro = A.prologue, epi = A.epilogue;
@@ -807,8 +812,8 @@ extern "C" int smlm_decode_linear(const smlm_linear_args *a, void *stream) {
     if ((A.n_split > 0 && (!A.out || A.out_stride < A.n_split || A.out_stride % 4 || (uintptr_t)A.out % 8)) ||
         (A.n_split < A.N && (!A.out2 || A.out2_stride < A.N - A.n_split || A.out2_stride % 4 || (uintptr_t)A.out2 % 8)))
       return fail(SMLM_EINVAL, "smlm_decode_linear: out / out2 missing, misaligned or with a short row stride");
-    if (A.w2 ? A.n_split < 16 || A.n_split >= A.N || !aligned16(A.w2) : A.bias2 != nullptr)
-      return fail(SMLM_EINVAL, "smlm_decode_linear: w2 (16-byte aligned) needs 0 < n_split < N; bias2 needs w2");
+    if (second.w && (A.n_split < 16 || A.n_split >= A.N || !aligned16(second.w)))
+      return fail(SMLM_EINVAL, "smlm_decode_linear: w2 (16-byte aligned) needs 0 < n_split < N");
     if (A.n_affine > 0 && (!A.scale || !A.shift))
       return fail(SMLM_EINVAL, "smlm_decode_linear: n_affine > 0 needs scale and shift");
   } else if (epi == SMLM_LIN_SWIGLU) {
@@ -821,8 +826,8 @@ extern "C" int smlm_decode_linear(const smlm_linear_args *a, void *stream) {
     if (A.pos_advance && A.M == 0)
       return fail(SMLM_EINVAL, "smlm_decode_linear: pos_advance needs M >= 1 (an empty launch runs nothing)");
   }
-  if ((A.w2 || A.bias2) && (epi != SMLM_LIN_STORE || pro != SMLM_LIN_PLAIN))
-    return fail(SMLM_EINVAL, "smlm_decode_linear: w2 and bias2 belong to the PLAIN prologue and STORE epilogue");
+  if (second.w && (epi != SMLM_LIN_STORE || pro != SMLM_LIN_PLAIN))
+    return fail(SMLM_EINVAL, "smlm_decode_linear: w2 belongs to the PLAIN prologue and STORE epilogue");
   if (A.pos_advance && epi != SMLM_LIN_ARGMAX)
     return fail(SMLM_EINVAL, "smlm_decode_linear: pos_advance belongs to the ARGMAX epilogue");
   if (A.M == 0) return SMLM_OK;
@@ -831,6 +836,7 @@ extern "C" int smlm_decode_linear(const smlm_linear_args *a, void *stream) {
   // groups measured 1% slower per batch-64 decode step; 16-row groups re-read the 24.6 MB of lm_head weights 4x),
   // and the PLAIN prologue with the STORE epilogue: 8-row groups (group_rows)
   LinGrid lg;
+  lg.second = second;
   lg.mtb = epi == SMLM_LIN_ARGMAX && A.M > 16 ? kMaxTiles : 1;
   const int tb = group_rows(pro, epi, lg.mtb);
   const int cols_per_block = epi == SMLM_LIN_ARGMAX ? kArgCols : 16;
@@ -854,6 +860,21 @@ extern "C" int smlm_decode_linear(const smlm_linear_args *a, void *stream) {
   else if (pro == SMLM_LIN_EMBED_RMSNORM) launch_linear_pro<SMLM_LIN_EMBED_RMSNORM>(A, lg, s);
   else launch_linear_pro<SMLM_LIN_EMBED_ARGMAX>(A, lg, s);
   return launch_status("smlm_decode_linear");
+}
+
+}  // namespace
+}  // namespace smlm
+
+extern "C" int smlm_linear_argmax_blocks(int N) { return N <= 0 ? 0 : (N + smlm::kArgCols - 1) / smlm::kArgCols; }
+
+extern "C" int smlm_decode_linear(const smlm_linear_args *a, void *stream) {
+  return smlm::decode_linear(a, {}, stream);
+}
+
+extern "C" int smlm_decode_linear_pair(const smlm_linear_args *a, const void *w2, const void *bias2, void *stream) {
+  using namespace smlm;
+  if (!w2) return fail(SMLM_EINVAL, "smlm_decode_linear_pair: null w2");
+  return decode_linear(a, {w2, bias2}, stream);
 }
 
 extern "C" int smlm_argmax_finish(const uint64_t *partial, int64_t partial_stride, int nblk, int64_t M, int64_t *pos,

@@ -33,7 +33,6 @@ class LinearArgs(ctypes.Structure):
         ("out2_stride", _i64), ("partial", _p), ("partial_stride", _i64), ("delta_parts", _i),
         ("tok_partial", _p), ("tok_partial_stride", _i64), ("tok_blocks", _i), ("tok_out", _p), ("hist", _p),
         ("hist_stride", _i64), ("hist_len", _i64), ("pos", _p), ("pos_advance", _p),
-        ("w2", _p), ("bias2", _p),
     ]
 
 # name -> (restype, argtypes); every function declared in include/smlm_pkm.h
@@ -63,6 +62,7 @@ EXPORTS = {
     "smlm_attention_backward": (_i, [_p] * 9 + [_i64, _p, _p, _i, _i, _i, _p, _i64, _i, _i, _i, _p]),
     "smlm_linear_argmax_blocks": (_i, [_i]),
     "smlm_decode_linear": (_i, [ctypes.POINTER(LinearArgs), _p]),
+    "smlm_decode_linear_pair": (_i, [ctypes.POINTER(LinearArgs), _p, _p, _p]),
     "smlm_argmax_finish": (_i, [_p, _i64, _i, _i64, _p, _p, _p, _i64, _i64, _i, _p]),
     "smlm_pkm_select_backward": (_i, [_p, _p, _p, _p, _i, _i64, _i, _i, _i, _p, _p, _p]),
     "smlm_score_keys_grad": (_i, [_p, _p, _p, _i64, _i, _i, _i, _p, _i, _p]),

@@ -657,12 +657,10 @@ def decode_linear(weight, x=None, *, delta=None, norm=None, tok=None, emb=None, 
                              "a multiple, without n_split, swiglu or argmax")
         n_split, n1 = N, N
         N += weight2.shape[0]
-        args.w2 = weight2.data_ptr()
         if bias2 is not None:
             if bias2.dtype != torch.bfloat16 or bias2.numel() != weight2.shape[0]:
                 raise ValueError("decode_linear: bias2 must be (N2,) bf16")
             bias2 = bias2.contiguous()
-            args.bias2 = bias2.data_ptr()
         keep += [weight2, bias2]
     else:
         n1 = N
@@ -777,7 +775,11 @@ def decode_linear(weight, x=None, *, delta=None, norm=None, tok=None, emb=None, 
         if out2 is not None:
             args.out2, args.out2_stride = out2.data_ptr(), N - split
         res = out1 if n_split is None else (out1, out2)
-    rc = _lib.lib().smlm_decode_linear(ctypes.byref(args), _stream(weight))
+    if weight2 is None:
+        rc = _lib.lib().smlm_decode_linear(ctypes.byref(args), _stream(weight))
+    else:
+        rc = _lib.lib().smlm_decode_linear_pair(ctypes.byref(args), weight2.data_ptr(),
+                                                None if bias2 is None else bias2.data_ptr(), _stream(weight))
     _lib.check(rc, "smlm_decode_linear")
     del keep
     return (x_out, res) if write_x else res
