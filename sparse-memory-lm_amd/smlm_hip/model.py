@@ -9,6 +9,7 @@ except the single-token decode step over the static cache, whose RoPE + cache wr
 config loads as is.
 """
 import math
+import weakref
 from dataclasses import asdict, dataclass, field
 
 import torch
@@ -529,12 +530,39 @@ class Transformer(nn.Module):
 
     def _decoder(self, B, max_len, device):
         key = (B, max_len, str(device), torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda"))
-        if key not in self._decoders:
-            self._decoders[key] = _StepDecoder(self, B, max_len, device)
-        return self._decoders[key]
+        dec = self._decoders.get(key)
+        if dec is None or dec._model() is None:     # a shallow copy shares them with a model that may be gone
+            dec = self._decoders[key] = _StepDecoder(self, B, max_len, device)
+        return dec
 
 
-class _FusedDecodeStep:
+class _KeptByModel:
+    """What a model keeps of its decoding, holding the model weakly: in a reference cycle a dropped model, its table, its
+    caches and its captured graphs would stay until Python's cyclic collector runs, and a graph that the collector
+    destroys while another one is being captured ends the process."""
+
+    def __init__(self, model):
+        self._model = weakref.ref(model)
+
+    @property
+    def model(self):
+        model = self._model()
+        if model is None:
+            raise ReferenceError(f"{type(self).__name__}: its model no longer exists")
+        return model
+
+    def __getstate__(self):             # copies and pickles of a model take its decoders along
+        state = dict(self.__dict__, model=self.model)
+        del state["_model"]
+        return state
+
+    def __setstate__(self, state):
+        state = dict(state)
+        self._model = weakref.ref(state.pop("model"))
+        self.__dict__.update(state)
+
+
+class _FusedDecodeStep(_KeptByModel):
     """One greedy decode step of a bf16 model on the fused decode kernels of smlm_hip.kernels.  Per dense block
         [residual add + attn_norm + wqkv] [RoPE + cache write + attention] [wo]
         [residual add + ffn_norm + w13 + SwiGLU] [w2]
@@ -596,7 +624,7 @@ class _FusedDecodeStep:
         return True
 
     def __init__(self, model):
-        self.model = model
+        super().__init__(model)
         self._tag = None
         self._prepare()
 
@@ -681,7 +709,7 @@ class _FusedDecodeStep:
         return None
 
 
-class _StepDecoder:
+class _StepDecoder(_KeptByModel):
     """Static buffers and the captured graphs of one decode step and of runs of `run_lengths` steps in a row for
     batch B, sequences up to max_len.  A step reads its position and token from device memory and advances them
     itself, so a run of steps is one graph replay: the replay boundary (about 15 us on MI355X) is paid once per
@@ -701,7 +729,8 @@ class _StepDecoder:
         cfg = model.cfg
         if max_len > cfg.max_seq_len:
             raise ValueError(f"prompt + new tokens = {max_len} exceed max_seq_len = {cfg.max_seq_len}")
-        self.model, self.B, self.max_len = model, B, max_len
+        super().__init__(model)
+        self.B, self.max_len = B, max_len
         dtype = model.tok_emb.weight.dtype
         if torch.is_autocast_enabled("cuda"):
             dtype = torch.get_autocast_dtype("cuda")
