@@ -130,6 +130,7 @@ def chained_launch_us(dev, numel=384, kernels=264, replays=40):
     captured decode step pays whatever its work; 262,144 values spread one kernel over the whole chip.
     264 = 8 decode steps of 33 kernels (the graph length does not change the per-kernel floor)."""
     import torch
+    from smlm_hip.capture import capture
     x = torch.zeros(numel, dtype=torch.float32, device=dev)
     side = torch.cuda.Stream(dev)
     side.wait_stream(torch.cuda.current_stream(dev))
@@ -138,7 +139,7 @@ def chained_launch_us(dev, numel=384, kernels=264, replays=40):
             x.add_(1.0)
     torch.cuda.current_stream(dev).wait_stream(side)
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
+    with capture(graph):
         for _ in range(kernels):
             x.add_(1.0)
     return 1000.0 * event_time_ms(graph.replay, replays) / kernels

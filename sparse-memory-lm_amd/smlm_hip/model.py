@@ -17,6 +17,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from . import kernels
+from .capture import capture
 from .engram import EngramMemory, NgramHash
 from .pkm import ProductKeyMemory, inference_tables, state_tag, state_tensors
 from .recording import ordinary, records, unhooked
@@ -460,7 +461,7 @@ class Transformer(nn.Module):
                     self(static_idx)
             torch.cuda.current_stream().wait_stream(side)
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph), ctx:
+            with capture(graph), ctx:
                 static_out = self(static_idx)
             entry = self._fwd_graphs[key] = (graph, static_idx, static_out)
         graph, static_idx, static_out = entry
@@ -822,14 +823,14 @@ class _StepDecoder(_KeptByModel):
             c.extra.update(extra)
         del saved, kv
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph), ctx:
+        with capture(graph), ctx:
             self._step()
         self.graph = graph
         self.graph_runs = {}
         for k in self.run_lengths:
             if k > 1:
                 run = torch.cuda.CUDAGraph()
-                with torch.cuda.graph(run), ctx:
+                with capture(run), ctx:
                     for _ in range(k):
                         self._step()
                 self.graph_runs[k] = run

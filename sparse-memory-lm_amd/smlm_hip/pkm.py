@@ -25,6 +25,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from . import kernels
+from .capture import capture
 from .recording import ordinary, records, unhooked
 from .sparse_values import check_impl, row_sparse_embedding_bag
 
@@ -296,7 +297,7 @@ class ProductKeyMemory(nn.Module):
                     self._forward(static_x)
             torch.cuda.current_stream().wait_stream(side)
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph), ctx:
+            with capture(graph), ctx:
                 static_out = self._forward(static_x)
             self._graph = (tag, graph, static_x, static_out)
         _, graph, static_x, static_out = self._graph
