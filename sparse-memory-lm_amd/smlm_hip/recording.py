@@ -1,6 +1,7 @@
 """When a kernel may stand in for a sequence of PyTorch ops that other machinery could be watching."""
 import torch
 from torch.autograd import forward_ad
+from torch.nn.modules import module as nn_module
 
 
 def ordinary(*tensors):
@@ -14,9 +15,12 @@ def ordinary(*tensors):
 
 
 def unhooked(*modules):
-    """Whether these modules' calls do nothing but their forward (no hooks), so that a kernel may read their weights."""
-    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                   for m in modules)
+    """Whether these modules' calls do nothing but their forward (no hooks of their own and none on all modules), so that a
+    kernel may read their weights."""
+    return not (nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks
+                or nn_module._global_backward_hooks or nn_module._global_backward_pre_hooks
+                or any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                       for m in modules))
 
 
 def records(*tensors):

@@ -587,3 +587,19 @@ def test_memory_layer_small_batches_of_any_layout(layout):
          "column stride": flat[:5 * 128].view(5, 64, 2)[..., 0]}[layout]
     got, ref = m(x).float(), m(x.contiguous().clone()).float()
     assert got.shape == ref.shape and float((got - ref).norm()) <= 0.1 * float(ref.norm())
+
+
+@torch.no_grad()
+def test_memory_layer_small_batches_under_a_global_hook():
+    """A hook on every module sees the layer's projections also at a few rows."""
+    from torch.nn.modules.module import register_module_forward_hook
+
+    from smlm_hip.pkm import ProductKeyMemory
+    m = ProductKeyMemory(64, 64, n_keys=64, heads=2, knn=8, k_dim=64).to(DEV).eval().to(torch.bfloat16)
+    x, seen = torch.randn(4, 64, device=DEV, dtype=torch.bfloat16), []
+    handle = register_module_forward_hook(lambda mod, args, out: seen.append(mod))
+    try:
+        m(x)
+    finally:
+        handle.remove()
+    assert {m.query_proj, m.swilu_proj, m.value_proj} <= set(seen)

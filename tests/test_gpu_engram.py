@@ -255,3 +255,18 @@ def test_engram_module_takes_the_kernel_or_the_ops():
         with torch.autograd.forward_ad.dual_level():
             assert count(b, h.bfloat16(), rows)[1] == 0
     assert EngramMemory.gated_value is ops
+
+
+def test_engram_module_under_a_global_hook():
+    """A hook on every module sees the norms and the convolution."""
+    note("engram module under a global hook")
+    from torch.nn.modules.module import register_module_forward_hook
+    m = EngramMemory(64, 16, 24, 53).to(DEV)
+    h, rows, seen = torch.randn(2, 40, 64, device=DEV), torch.randint(0, 53, (2, 40, 16), device=DEV), []
+    handle = register_module_forward_hook(lambda mod, args, out: seen.append(mod))
+    try:
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            m(h, rows)
+    finally:
+        handle.remove()
+    assert {m.h_norm, m.k_norm, m.v_norm, m.conv} <= set(seen)
