@@ -1,9 +1,12 @@
 """When a kernel may stand in for PyTorch ops that something else is watching (smlm_hip.recording)."""
 import pytest
+import torch
 from torch import nn
 from torch.nn.modules import module as nn_module
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
-from smlm_hip.recording import unhooked
+from smlm_hip.recording import ordinary, unhooked
 
 
 def _nothing(*args, **kwargs):
@@ -30,3 +33,36 @@ def test_every_module_is_called_under_a_global_hook(register):
     finally:
         handle.remove()
     assert unhooked(plain)
+
+
+class _Functions(TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+class _Dispatches(TorchDispatchMode):
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("mode", [_Functions, _Dispatches])
+def test_nothing_is_ordinary_under_a_mode(mode):
+    x = torch.zeros(2)
+    with mode():
+        assert not ordinary(x)
+        with torch.device("cpu"):
+            assert not ordinary(x)
+    assert ordinary(x)
+
+
+def test_a_default_device_is_ordinary():
+    """torch.device as a context and set_default_device are function modes that touch factory calls only."""
+    x = torch.zeros(2)
+    with torch.device("cpu"):
+        assert ordinary(x)
+    torch.set_default_device("cpu")
+    try:
+        assert ordinary(x)
+    finally:
+        torch.set_default_device(None)
+    assert ordinary(x)
