@@ -47,12 +47,15 @@ class _SubkeyScores(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, keys):
+        ctx.set_materialize_grads(False)                   # a half that was not used comes as None
         k = kernels._aligned(keys.detach().to(q.dtype))    # bf16 keys may be a view into a flat buffer
         ctx.save_for_backward(q, keys, k)
         return kernels.pk_scores(kernels._aligned(q), k)
 
     @staticmethod
     def backward(ctx, g1, g2):
+        if g1 is None and g2 is None:
+            return None, None
         q, keys, k = ctx.saved_tensors
         if torch.is_grad_enabled():
             out, grads = zip(*((s, g) for s, g in zip(_score_ops(q, keys.to(q.dtype)), (g1, g2)) if g is not None))
