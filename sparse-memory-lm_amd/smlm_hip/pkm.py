@@ -404,11 +404,20 @@ class ProductKeyMemory(nn.Module):
 
     SMALL_BATCH = 64      # rows up to which the projections run on the decode step's kernel
 
+    def _small_batch_rows(self):
+        """SMALL_BATCH, or less in a wide layer: the kernel reads the three weights once per 8 rows, which beats the library's
+        launches while they are small.  Captured layer, library -> kernel (us): 64 rows of 0.7 M weights (384 wide, 1,024
+        query columns) 32 -> 21, of 4.2 M (1,024 wide, 2,048) 48 -> 38, of 6.3 M (1,024 wide, 4,096) 55 -> 51, but of
+        8.1 M (1,536 wide, 2,048) 47 -> 57 and of 10.5 M (1,024 wide, 8,192) 64 -> 73; 32 rows of 16.8 M (2,048 wide, 4,096)
+        61 -> 63; 16 rows of 16.8 M 56 -> 46 and of 25.2 M (2,048 wide, 8,192) 72 -> 69, the widest measured."""
+        weights = self.d_in * (self.heads * self.k_dim + self.v_dim) + self.v_dim * self.d_out
+        return min(self.SMALL_BATCH, 64 if weights <= 6 << 20 else 16 if weights <= 24 << 20 else 0)
+
     def _small_batch(self, x):
         """Whether a no-grad bf16 call's projections run on kernels.decode_linear: few rows, where the library's products
-        and the query's affine are four launches for a few microseconds of work, here two (1 / 16 / 64 tokens, 1024
-        sub-keys, eager: 138 / 124 / 123 -> 79 us; captured and waited for: 63-66 / 60-62 / 70 -> 56-60)."""
-        if not 0 < x.shape[0] <= self.SMALL_BATCH or not self.swilu:
+        and the query's affine are four launches for a few microseconds of work, here two (16 tokens, 384 wide, 1,024 query
+        columns: eager 131 -> 88 us, captured 26 -> 19)."""
+        if not 0 < x.shape[0] <= self.SMALL_BATCH or not self.swilu or x.shape[0] > self._small_batch_rows():
             return False
         # the kernel reads rows of its own, 16 bytes at a time: a repeated row (expand) or one off its alignment (a slice)
         # stays with the modules

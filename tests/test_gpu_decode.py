@@ -531,6 +531,23 @@ def test_decode_linear_of_two_weights(M, K_in, N1, N2, biased):
             K.decode_linear(ws[0], x, **bad)
 
 
+@pytest.mark.parametrize("M", [1, 16, 64])
+@pytest.mark.parametrize("K_in", [512, 1024, 1056, 2048])
+def test_decode_linear_of_two_wide_weights(M, K_in):
+    """The wider register layouts, up to the widest: the same bits as a launch for each weight, and the products
+    themselves."""
+    note(f"decode_linear two wide weights M={M} K={K_in}")
+    g = torch.Generator().manual_seed(M + K_in)
+    x = bf(torch.randn(M, K_in, generator=g))
+    ws = [bf(torch.randn(n, K_in, generator=g) * K_in ** -0.5) for n in (272, 80)]
+    bs = [bf(torch.randn(n, generator=g)) for n in (272, 80)]
+    dx, dws, dbs = x.to(DEV), [w.to(DEV) for w in ws], [b.to(DEV) for b in bs]
+    got = K.decode_linear(dws[0], dx, bias=dbs[0], weight2=dws[1], bias2=dbs[1])
+    for y, w, b, dw, db in zip(got, ws, bs, dws, dbs):
+        assert torch.equal(y, K.decode_linear(dw, dx, bias=db))
+        assert_bf16_close(y, x.double() @ w.double().T + b.double(), "two wide weights")
+
+
 @torch.no_grad()
 def test_memory_layer_small_batches_take_the_decode_kernel():
     """Up to 64 rows in bf16 the layer's projections run on the decode step's kernel, with the query's affine and
