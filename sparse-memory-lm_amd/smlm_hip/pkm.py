@@ -434,7 +434,8 @@ class ProductKeyMemory(nn.Module):
             if not (type(lin) is nn.Linear and w.dtype == torch.bfloat16 and w.device == x.device and w.is_contiguous()
                     and w.data_ptr() % 16 == 0 and (b is None or (b.dtype == torch.bfloat16 and b.device == x.device))):
                 return False
-        return unhooked(*lins) and ordinary(x) and not records(x, *(lin.weight for lin in lins))
+        operands = [t for lin in lins for t in (lin.weight, lin.bias)]
+        return unhooked(*lins) and ordinary(x, *operands) and not records(x, *operands)
 
     def _forward(self, x):
         if torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in self.parameters())):

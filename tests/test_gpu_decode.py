@@ -620,3 +620,28 @@ def test_memory_layer_small_batches_under_a_global_hook():
     finally:
         handle.remove()
     assert {m.query_proj, m.swilu_proj, m.value_proj} <= set(seen)
+
+
+class _Subclass(torch.Tensor):
+    pass
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("part", ["weight", "bias"])
+@pytest.mark.parametrize("name", ["query_proj", "swilu_proj", "value_proj"])
+def test_memory_layer_small_batches_of_subclassed_weights(name, part):
+    """A projection whose parameter is a tensor subclass (which may hold its values elsewhere) is called."""
+    from smlm_hip.pkm import ProductKeyMemory
+    torch.manual_seed(0)
+    m = ProductKeyMemory(64, 64, n_keys=64, heads=2, knn=8, k_dim=64).to(DEV).eval().to(torch.bfloat16)
+    assert m._small_batch(torch.zeros(4, 64, device=DEV, dtype=torch.bfloat16))
+    lin = getattr(m, name)
+    setattr(lin, part, torch.nn.Parameter(getattr(lin, part).detach().as_subclass(_Subclass)))
+    assert type(getattr(lin, part)) is _Subclass
+    x, called = torch.randn(4, 64, device=DEV, dtype=torch.bfloat16), []
+    real = K.decode_linear
+    K.decode_linear = lambda *a, **kw: (called.append(1), real(*a, **kw))[1]
+    try:
+        assert m(x).shape == (4, 64) and not called
+    finally:
+        K.decode_linear = real

@@ -270,3 +270,25 @@ def test_engram_module_under_a_global_hook():
     finally:
         handle.remove()
     assert {m.h_norm, m.k_norm, m.v_norm, m.conv} <= set(seen)
+
+
+class _Subclass(torch.Tensor):
+    pass
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("name", ["w_k", "w_v"])
+def test_engram_module_with_subclassed_projection_weights(name):
+    """A projection whose weight is a tensor subclass (which may hold its values elsewhere) is called as a module."""
+    note(f"engram module with a subclassed {name}")
+    m = EngramMemory(128, 16, 24, 53).to(DEV, torch.bfloat16)
+    lin, seen = getattr(m, name), []
+    lin.weight = torch.nn.Parameter(lin.weight.detach().as_subclass(_Subclass))
+    assert type(lin.weight) is _Subclass
+    real = K.prompt_linear
+    K.prompt_linear = lambda x, w, *a: (seen.append(type(w)), real(x, w, *a))[1]
+    try:
+        m(torch.randn(2, 128, 128, device=DEV).bfloat16(), torch.randint(0, 53, (2, 128, 16), device=DEV))
+    finally:
+        K.prompt_linear = real
+    assert _Subclass not in seen
