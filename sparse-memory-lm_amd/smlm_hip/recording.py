@@ -23,12 +23,12 @@ def ordinary(*tensors):
 
 
 def unhooked(*modules):
-    """Whether these modules' calls do nothing but their forward (no hooks of their own and none on all modules), so that a
-    kernel may read their weights."""
+    """Whether these modules' calls do nothing but their class's forward (no hooks of their own, none on all modules, no
+    forward put on the module), so that a kernel may read their weights."""
     return not (nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks
                 or nn_module._global_backward_hooks or nn_module._global_backward_pre_hooks
                 or any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                       for m in modules))
+                       or "forward" in m.__dict__ for m in modules))
 
 
 def records(*tensors):

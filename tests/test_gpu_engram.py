@@ -292,3 +292,30 @@ def test_engram_module_with_subclassed_projection_weights(name):
     finally:
         K.prompt_linear = real
     assert _Subclass not in seen
+
+
+class _Doubled(torch.nn.Linear):
+    def forward(self, x):
+        return 2 * super().forward(x)
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("how", ["class", "instance"])
+def test_engram_module_with_a_projection_of_its_own(how):
+    """A projection with another forward than nn.Linear's, by its class or put on the module, is called: the result of
+    the doubled weight, up to bf16."""
+    note(f"engram module with a projection of its own: {how}")
+    torch.manual_seed(2)
+    m = EngramMemory(128, 16, 24, 53).to(DEV, torch.bfloat16)
+    m.conv.weight.normal_(std=0.3)
+    h, rows = torch.randn(2, 128, 128, device=DEV).bfloat16(), torch.randint(0, 53, (2, 128, 16), device=DEV)
+    plain, w = m.w_v, m.w_v.weight.detach().clone()
+    plain.weight.mul_(2)
+    ref = m(h, rows).float()
+    plain.weight.copy_(w)
+    if how == "class":
+        m.w_v = _Doubled(384, 128, bias=False).to(DEV, torch.bfloat16)
+        m.w_v.weight.copy_(w)
+    else:
+        plain.forward = lambda x: 2 * torch.nn.Linear.forward(plain, x)
+    assert float((m(h, rows).float() - ref).norm()) <= 2 ** -6 * float(ref.norm())

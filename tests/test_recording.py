@@ -35,6 +35,14 @@ def test_every_module_is_called_under_a_global_hook(register):
     assert unhooked(plain)
 
 
+def test_a_module_with_a_forward_of_its_own_is_called():
+    watched = nn.Linear(2, 2)
+    watched.forward = _nothing
+    assert not unhooked(watched)
+    del watched.forward
+    assert unhooked(watched)
+
+
 class _Functions(TorchFunctionMode):
     def __torch_function__(self, func, types, args=(), kwargs=None):
         return func(*args, **(kwargs or {}))
