@@ -65,6 +65,9 @@ MAX_N_KEYS = 65536    # sub-key indices fit the 16-bit index field of the select
 MAX_KNN = 128         # the selection's result lists (csrc/pkm_select.hip: kMaxKnnGen)
 
 
+SCORE_MAX_HEADS = 32768     # most heads of pk_scores and score_keys_grad
+
+
 def pk_scores(q, keys):
     """q (N, H, k_dim), keys (H, 2, NK, k_dim/2) of the same dtype (bf16 or fp32) -> s1, s2 (N, H, NK) of that
     dtype: s1[n,h,k] = q[n,h,:half] . keys[h,0,k], s2 with q[n,h,half:] and keys[h,1] (smlm/pkm.py:117-123).
@@ -861,7 +864,7 @@ class PKSelect(torch.autograd.Function):
 
 def score_keys_grad_supported(N, H, NK, half):
     """Whether score_keys_grad takes these shapes: whole 16-byte chunks, byte offsets of 32 bits."""
-    return N > 0 and NK % 8 == 0 and half % 8 == 0 and (N + 320) * H * max(NK, 2 * half) * 2 + 512 < 2 ** 31
+    return N > 0 and 0 < H <= SCORE_MAX_HEADS and NK % 8 == 0 and half % 8 == 0 and (N + 320) * H * max(NK, 2 * half) * 2 + 512 < 2 ** 31
 
 
 def score_keys_grad(g1, g2, q, keys_shape, dtype):
@@ -881,6 +884,11 @@ def score_keys_grad(g1, g2, q, keys_shape, dtype):
                                          q.data_ptr(), N, H, NK, half, dk.data_ptr(), _DT[dtype], _stream(q))
     _lib.check(rc, "smlm_score_keys_grad")
     return dk
+
+
+def query_norm_supported(N, C):
+    """Whether query_norm_backward takes these shapes."""
+    return N >= 2 and C % 8 == 0 and 8 <= C <= 1 << 20
 
 
 def query_norm_backward(g, x, weight, mean, invstd):

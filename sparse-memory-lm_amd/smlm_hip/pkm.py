@@ -351,7 +351,7 @@ class ProductKeyMemory(nn.Module):
         stats = (bn.running_mean, bn.running_var) if bn.track_running_stats else (None, None)
         columns = (bn.weight, bn.bias, *stats)
         if (to_bf16 and type(bn) is nn.BatchNorm1d and bn.training and q.is_cuda and q.dtype == torch.bfloat16
-                and q.dim() == 2 and q.shape[0] > 1 and q.shape[1] % 8 == 0 and bn.affine and bn.momentum is not None
+                and q.dim() == 2 and kernels.query_norm_supported(*q.shape) and bn.affine and bn.momentum is not None
                 and unhooked(bn) and records(q, bn.weight, bn.bias) and not records(*stats)
                 and all(t is None or (t.dtype == torch.float32 and t.device == q.device and t.is_contiguous()
                                       and t.shape == (q.shape[1],)) for t in columns)
@@ -377,6 +377,7 @@ class ProductKeyMemory(nn.Module):
             q = q.to(torch.bfloat16)
         keys = self.keys
         if (q.is_cuda and q.dtype == torch.bfloat16 and q.numel() and (self.k_dim // 2) % 8 == 0
+                and self.heads <= kernels.SCORE_MAX_HEADS
                 and (keys.dtype == torch.bfloat16 or (keys.dtype == torch.float32 and _autocast_bf16(x)))
                 and keys.device == q.device and ordinary(q, keys)):
             s1, s2 = _SubkeyScores.apply(q, keys)
