@@ -333,7 +333,8 @@ class ProductKeyMemory(nn.Module):
     def _bn_affine(self):
         """fp32 (scale, shift) of the eval-mode BatchNorm, cached until its parameters or statistics change."""
         bn = self.query_norm
-        parts = (bn.running_mean, bn.running_var, bn.weight, bn.bias)
+        # torch's batch norm writes the statistics without a new version, but counts the batch
+        parts = (bn.running_mean, bn.running_var, bn.weight, bn.bias, bn.num_batches_tracked)
         tag = tuple((t.data_ptr(), t._version) if t is not None else None for t in parts)
         if self._bn_cache is None or self._bn_cache[0] != tag:
             inv = torch.rsqrt(bn.running_var.float() + bn.eps)
