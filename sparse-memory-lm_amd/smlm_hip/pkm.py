@@ -410,7 +410,7 @@ class ProductKeyMemory(nn.Module):
         """SMALL_BATCH, or less in a wide layer: the kernel reads the three weights once per 8 rows, which beats the library's
         launches while they are small.  Captured layer, library -> kernel (us): 64 rows of 0.7 M weights (384 wide, 1,024
         query columns) 32 -> 21, of 4.2 M (1,024 wide, 2,048) 48 -> 38, of 6.3 M (1,024 wide, 4,096) 55 -> 51, but of
-        8.1 M (1,536 wide, 2,048) 47 -> 57 and of 10.5 M (1,024 wide, 8,192) 64 -> 73; 32 rows of 16.8 M (2,048 wide, 4,096)
+        7.9 M (1,536 wide, 2,048) 47 -> 57 and of 10.5 M (1,024 wide, 8,192) 64 -> 73; 32 rows of 16.8 M (2,048 wide, 4,096)
         61 -> 63; 16 rows of 16.8 M 56 -> 46 and of 25.2 M (2,048 wide, 8,192) 72 -> 69, the widest measured."""
         weights = self.d_in * (self.heads * self.k_dim + self.v_dim) + self.v_dim * self.d_out
         return min(self.SMALL_BATCH, 64 if weights <= 6 << 20 else 16 if weights <= 24 << 20 else 0)
@@ -431,12 +431,13 @@ class ProductKeyMemory(nn.Module):
                 and self.d_out % 16 == 0 and (bn is None or not bn.training)
                 and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)):
             return False
+        operands = []
         for lin in lins:
             w, b = lin.weight, lin.bias
+            operands += (w, b)
             if not (type(lin) is nn.Linear and w.dtype == torch.bfloat16 and w.device == x.device and w.is_contiguous()
                     and w.data_ptr() % 16 == 0 and (b is None or (b.dtype == torch.bfloat16 and b.device == x.device))):
                 return False
-        operands = [t for lin in lins for t in (lin.weight, lin.bias)]
         return unhooked(*lins) and ordinary(x, *operands) and not records(x, *operands)
 
     def _forward(self, x):

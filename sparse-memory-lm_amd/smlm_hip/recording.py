@@ -25,10 +25,15 @@ def ordinary(*tensors):
 def unhooked(*modules):
     """Whether these modules' calls do nothing but their class's forward (no hooks of their own, none on all modules, no
     forward put on the module), so that a kernel may read their weights."""
-    return not (nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks
-                or nn_module._global_backward_hooks or nn_module._global_backward_pre_hooks
-                or any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                       or "forward" in m.__dict__ for m in modules))
+    if (nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks or nn_module._global_backward_hooks
+            or nn_module._global_backward_pre_hooks):
+        return False
+    for m in modules:
+        own = m.__dict__
+        if (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
+                or "forward" in own):
+            return False
+    return True
 
 
 def records(*tensors):
