@@ -287,11 +287,11 @@ int launch_flash(const void *q, const int64_t *qs, const void *k, const int64_t 
 // LDS reads: dQ^T = K^T dS^T, dK^T = Q^T dS, dV^T = dO^T P.  Scores, dP, P and dS in fp32; P and dS rounded to bf16 for
 // the products.  The first launch writes delta = <dO, y> per query for the second.  The epilogue undoes RoPE (a lane
 // holds both halves of a rotation pair) and writes the gradient of the qkv projection's rows (B, T, 3, H, hd).
-// As PyTorch ops (fp32 softmax over materialised scores, masks, copies, bmm and their gradients) a training pass of
-// the attention block over 4 x 1,024 tokens with 6 heads of 64 took 1,099 us (960 of kernels), now 337 (207: the
-// forward 27, this 58, the projections' library products the rest).  Bound by the walk's latency there (384
-// workgroups); 8 x 2,048 tokens 143 us, 629 TFLOP/s of the seven products.  128 own rows per workgroup: 64 against 55
-// us, equal at 8 x 2,048.
+// As PyTorch ops (fp32 softmax over materialised scores, masks, copies, bmm and their gradients) a training pass of the
+// attention block over 4 x 1,024 tokens with 6 heads of 64 took 960 us of kernels, now 207: the forward 27, this 58, the
+// projections' library products the rest (the pass 1,017 -> 471: the host's launches and autograd).  Bound by the walk's
+// latency there (384 workgroups); 8 x 2,048 tokens 143 us, 629 TFLOP/s of the seven products.  128 own rows per
+// workgroup: 64 against 55 us, equal at 8 x 2,048.
 struct AttnGradArgs {
   const uint16_t *q, *k, *v, *y, *dy;        // q, k (B, H, T, hd); v, y, dy with their strides over (b, h, t)
   int64_t vsb, vsh, vst, ysb, ysh, yst;      // y and dy share strides

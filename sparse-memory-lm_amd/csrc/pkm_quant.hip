@@ -83,12 +83,14 @@ __device__ __forceinline__ void argmax_step(float &best, int &bi) {
 
 // Bound by the row's read (1,536 bytes of fp32 for 384 codes).  quantize_kernel reads 4 bytes per lane, reads every
 // row twice, reduces over 64 lanes through LDS and divides 384 times by the IEEE sequence: 1,048,576 x 384 fp32 -> int8
-// took 1,004 us (2.0 TB/s); this kernel takes 355 us (5.7 TB/s, the rate of a copy).  Here 16 lanes hold a row as NC chunks of 4 columns each (16-byte loads, all in flight
-// before the first use, four rows per wavefront), the maximum takes four DPP steps, and the quotient is a product
-// with the row's correctly rounded reciprocal, corrected once by its fma residual, which is the IEEE quotient
-// (Markstein's theorem) unless something overflows or a term underflows: the scale's magnitude is at least 2^-24, the
-// quotients that do not round to code 0 are 0.5 .. 129, so no term that matters is subnormal; a scale that is not
-// finite (a row beyond 65504 x |lo|, or one that holds an infinity) takes the division itself.
+// took 1,004 us (2.0 TB/s); this kernel takes 355 us (5.7 TB/s, the rate of a copy).  Here 16 lanes hold a row as NC
+// chunks of 4 columns each (16-byte loads, all in flight before the first use, four rows per wavefront), the maximum
+// takes four DPP steps, and the quotient is a product with the row's correctly rounded reciprocal, corrected once by its
+// fma residual, which is the IEEE quotient (Markstein's theorem) unless something overflows or a term underflows: the
+// scale's magnitude is at least 2^-24, and the quotients that do not round to code 0 are 0.5 to 1.5 x |lo| (the row's
+// largest magnitude is |lo| times the scale before its rounding to fp16, which takes off less than a third even of a
+// subnormal one), so no term that matters is subnormal; a scale that is not finite (a row beyond 65504 x |lo|, or one that
+// holds an infinity) takes the division itself.
 // Q4: chunk c of the first half and the chunk D/2 columns later are the same lane's, so a byte's nibbles meet there.
 template <bool SRC_F32, bool Q4, int NC>
 __global__ void __launch_bounds__(256) quantize_rows_kernel(const void *__restrict__ src, int64_t rows, int D,
