@@ -14,7 +14,8 @@ the reference's power-of-two rule for it.
 
 A forward that autograd records (training) takes the reference's differentiable path with the HIP kernels where the
 reference uses its Triton ones (smlm/pkm.py:186-228): torch query projection and BatchNorm (its gradient on a kernel in
-bf16), sub-key scores by pk_scores in bf16 and by torch.einsum otherwise (the backward is library GEMMs), the selection and its backward on the kernels (kernels.PKSelect),
+bf16), sub-key scores by pk_scores in bf16 (the keys' gradient on a kernel, the query's by library GEMMs) and by
+torch.einsum otherwise, the selection and its backward on the kernels (kernels.PKSelect),
 and the values through the row-sparse bag (smlm_hip.sparse_values: fp32 accumulator + touched flags for
 LazyRowAdam) or, with value_grad="dense", F.embedding_bag.
 """
