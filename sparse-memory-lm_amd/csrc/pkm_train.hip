@@ -628,7 +628,12 @@ __global__ void __launch_bounds__(kTrainThreads) lazy_adam_kernel(AdamArgs A) {
 // 8,388,592 rows x 24, fp32 moments, 0.6% / 40% / all rows flagged 351 / 1,527 / 2,641 us, here 25 / 945 / 1,288 us
 // (bf16 343 / 1,517 / 2,959 -> 26 / 778 / 971; int8 439 / 2,969 / 6,819 -> 46 / 698 / 1,010).  Now bound by the flags
 // (one byte per row) or the flagged rows' cache lines.  The same scan over wide rows lost with most rows flagged
-// (1,048,576 x 384 fp32, all: 2,393 -> 2,478-2,560 us): its rows wait for the list.
+// (1,048,576 x 384 fp32, all: 2,393 -> 2,478-2,560 us): its rows wait for the list.  Towards 128 columns that shows too:
+// 1,000,000 x 128 with 1 / 40 / 70 / 100% of the rows flagged 75 / 328 / 528 / 719 us by a wavefront per row, here 12 /
+// 335 / 571 / 785 (bf16 71 / 297 / 421 / 528 -> 12 / 252 / 426 / 585; int8 87 / 415 / 617 / 795 -> 19 / 232 / 383 / 520).
+// A lazy step reads part of its table, so the list stays up to 128 columns; the host does not know the share.  Lists per
+// workgroup, the next rows' loads before this one's stores, another first row per wavefront, fewer wavefronts in flight:
+// 780-805 us with all rows flagged; 2 rows per scan 757, but 54 at 1%.
 constexpr int kScanMost = 256;
 template <int STATE, int G>
 __global__ void __launch_bounds__(kTrainThreads) lazy_adam_narrow_kernel(AdamArgs A) {
