@@ -863,8 +863,13 @@ class PKSelect(torch.autograd.Function):
 
 
 def score_keys_grad_supported(N, H, NK, half):
-    """Whether score_keys_grad takes these shapes: whole 16-byte chunks, byte offsets of 32 bits."""
-    return N > 0 and 0 < H <= SCORE_MAX_HEADS and NK % 8 == 0 and half % 8 == 0 and (N + 320) * H * max(NK, 2 * half) * 2 + 512 < 2 ** 31
+    """Whether score_keys_grad takes these shapes (whole 16-byte chunks, byte offsets of 32 bits) and is the faster one: it
+    walks the tokens once per 64 keys x 128 columns, so many tokens and narrow halves leave it few workgroups, where the
+    library splits them (H 1, 128 keys, half 32: 16,384 tokens 82 us against 84, 65,536 316 against 177; H 4, 256 keys,
+    half 256: 65,536 tokens 456 against 621, 131,072 927 against 1,089; H 1, 1,024 keys, half 256: 911 against 941 at
+    131,072, 1,822 against 1,551 at 262,144)."""
+    return (0 < N <= (131072 if half >= 256 else 16384) and 0 < H <= SCORE_MAX_HEADS and NK % 8 == 0 and half % 8 == 0
+            and (N + 320) * H * max(NK, 2 * half) * 2 + 512 < 2 ** 31)
 
 
 def score_keys_grad(g1, g2, q, keys_shape, dtype):

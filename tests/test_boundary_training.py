@@ -18,6 +18,14 @@ def test_the_keys_gradient_is_asked_for_what_it_takes(N, H, NK, half):
     assert kernels.score_keys_grad_supported(4096, 4, 1024, 256)
 
 
+@pytest.mark.parametrize("N,H,NK,half,taken", [(16384, 1, 128, 32, True), (16385, 1, 128, 32, False), (16384, 8, 1024, 248, True),
+                                               (65536, 4, 128, 248, False), (131072, 4, 256, 256, True),
+                                               (131073, 4, 256, 256, False)])
+def test_long_walks_of_the_keys_gradient_go_through_the_library(N, H, NK, half, taken):
+    """More tokens than its few workgroups walk faster than the library's split products."""
+    assert kernels.score_keys_grad_supported(N, H, NK, half) == taken
+
+
 def test_the_scores_are_asked_for_what_they_take():
     lib, most = _lib.lib(), kernels.SCORE_MAX_HEADS
     assert lib.smlm_pkm_score(FAKE, 16 * (most + 1), FAKE, _lib.BF16, 0, most + 1, 8, 8, FAKE, FAKE, None) == _lib.EINVAL
