@@ -44,7 +44,7 @@ def test_the_query_norm_gradient_is_asked_for_what_it_takes(N, C):
 @pytest.mark.parametrize("N,C,taken", [(16384, 8, True), (16385, 8, False), (131072, 64, True), (131073, 64, False),
                                        (246000, 120, False), (1 << 20, 128, True)])
 def test_tall_narrow_query_norms_go_through_torch(N, C, taken):
-    """More rows than few columns leave lanes for."""
+    """Few columns leave most lanes of the kernel idle."""
     assert kernels.query_norm_supported(N, C) == taken
 
 
